@@ -389,26 +389,6 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
   if (g == 0 && (!RAG || qrow < S)) a.lse[(int64_t)bh * S + qrow] = (m_run + fast_log2(l_tot)) * kLn2;
 }
 
-// Compute units of the device `st` launches on (cached per device), the size
-// of one dispatch round of the grid ordering; 0 when unknown or not a multiple
-// of the 8 XCDs.  Calls may come from several host threads at once (the
-// forward from the caller's, the backward from autograd's): the cache entries
-// are atomics, and a race only makes two threads store the same value.
-int cu_count(hipStream_t st) {
-  static std::atomic<int> cache[64];
-  int dev = -1;
-  if (hipStreamGetDevice(st, &dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int n = cache[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      cus = 0;
-    n = (cus > 0 && cus % 8 == 0) ? cus : -1;
-    cache[dev].store(n, std::memory_order_relaxed);
-  }
-  return n > 0 ? n : 0;
-}
-
 template <typename E, int D, int DP = D, bool RAG = false>
 hipError_t launch_fwd_d(const AttnArgs& a, hipStream_t st) {
   const int n_qtiles = (a.S + FwdCfg<D>::BQ - 1) / FwdCfg<D>::BQ;
@@ -439,6 +419,26 @@ hipError_t launch_fwd_e(const AttnArgs& a, hipStream_t st) {
 }
 
 }  // namespace
+
+// Compute units of the device `st` launches on (cached per device), the size
+// of one dispatch round of the grid ordering; 0 when unknown or not a multiple
+// of the 8 XCDs.  Calls may come from several host threads at once (the
+// forward from the caller's, the backward from autograd's): the cache entries
+// are atomics, and a race only makes two threads store the same value.
+int cu_count(hipStream_t st) {
+  static std::atomic<int> cache[64];
+  int dev = -1;
+  if (hipStreamGetDevice(st, &dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      cus = 0;
+    n = (cus > 0 && cus % 8 == 0) ? cus : -1;
+    cache[dev].store(n, std::memory_order_relaxed);
+  }
+  return n > 0 ? n : 0;
+}
 
 bool mfma_supports(int dtype, int D, int S) {
   return (dtype == 1 || dtype == 2) && S > 0 && (D == 16 || D == 32 || D == 64 || D == 128);

@@ -3,9 +3,9 @@
 // Same algorithm as the MFMA kernels (online-softmax forward with saved
 // log-sum-exp, FlashAttention-2 backward), 8 lanes (4 at D = 16) per query row
 // (forward, dQ) or per key row (dK/dV), with 64-row K/V (or Q/dO) tiles staged
-// in LDS as fp32.  Used for fp32 tensors (no rounding anywhere: fp32 in, fp32
-// math, fp32 out), for any S (tails are masked) and for head dims / strides the
-// MFMA kernels do not cover.  Counterparts: `_attn_fwd` (core/myFlashAttn.py:447-728),
+// in LDS as fp32.  Used for 16-bit tensors whose rows are not 16-byte aligned,
+// which the MFMA kernels' loads cannot take, for any S (tails are masked).
+// Counterparts: `_attn_fwd` (core/myFlashAttn.py:447-728),
 // `_attn_bwd_LoopKV` (:1069-1317) and `_attn_bwd_LoopQ` (:795-1066).
 #include "mi_device.h"
 #include "mi_kernels.h"
@@ -376,19 +376,16 @@ hipError_t dq_t(const AttnArgs& a, hipStream_t st) {
 bool valu_supports(int D) { return D == 16 || D == 32 || D == 64 || D == 128; }
 
 hipError_t launch_attn_fwd_valu(int dtype, const AttnArgs& a, hipStream_t st) {
-  if (dtype == 0) return fwd_t<0>(a, st);
   if (dtype == 1) return fwd_t<1>(a, st);
   return fwd_t<2>(a, st);
 }
 
 hipError_t launch_attn_bwd_dkdv_valu(int dtype, const AttnArgs& a, hipStream_t st) {
-  if (dtype == 0) return dkdv_t<0>(a, st);
   if (dtype == 1) return dkdv_t<1>(a, st);
   return dkdv_t<2>(a, st);
 }
 
 hipError_t launch_attn_bwd_dq_valu(int dtype, const AttnArgs& a, hipStream_t st) {
-  if (dtype == 0) return dq_t<0>(a, st);
   if (dtype == 1) return dq_t<1>(a, st);
   return dq_t<2>(a, st);
 }

@@ -1,8 +1,8 @@
 // capi.hip — the extern "C" surface declared in include/mi_attn.h.
 //
 // Validates every argument before anything is enqueued, picks the kernel
-// family (bf16/f16 MFMA when the shape and alignment allow it, exact-fp32
-// VALU otherwise) and reports failures as status codes plus a per-thread
+// family (bf16/f16 MFMA for 16-byte aligned rows, exact-fp32 VALU for other
+// rows of those types, fp32 MFMA for fp32) and reports failures as status codes plus a per-thread
 // message.  No allocation and no synchronisation.  Global mutable state: the
 // thread-local error text, and the forward's per-device cache of the compute
 // unit count (atomic entries, written once per device with the same value).
@@ -216,6 +216,8 @@ mi_status mi_attn_fwd(mi_dtype dtype, int B, int H, int S, int D, int causal, fl
     return launched(mi::launch_attn_fwd_mfma(dtype, a, (hipStream_t)stream), "attn_fwd_mfma");
   if (!mi::valu_supports(D))
     return fail(MI_ERR_UNSUPPORTED, "head dim %d not supported (16, 32, 64, 128)", D);
+  if (dtype == MI_F32)
+    return launched(mi::launch_attn_fwd_f32(a, al, (hipStream_t)stream), "attn_fwd_f32");
   return launched(mi::launch_attn_fwd_valu(dtype, a, (hipStream_t)stream), "attn_fwd_valu");
 }
 
@@ -328,6 +330,19 @@ static mi_status grads_impl(mi_dtype dtype, int B, int H, int S, int D, int caus
     if (fuse_rope) a.rope = *rope;
     if ((st = launched(mi::launch_attn_bwd_mfma(dtype, a, (hipStream_t)stream),
                        "attn_bwd_mfma")) != MI_OK || !rope || fuse_rope)
+      return st;
+  } else if (dtype == MI_F32) {
+    mi::AttnArgs a = grad_args(B, H, S, D, causal, scale, q, q_strides, k, k_strides, v,
+                               v_strides, dout, dout_strides, lse, ws);
+    a.dq = targ(dq, dq_strides);
+    a.dk = targ(dk, dk_strides);
+    a.dv = targ(dv, dv_strides);
+    const bool al = aligned16(q, q_strides, 4) && aligned16(k, k_strides, 4) &&
+                    aligned16(v, v_strides, 4) && aligned16(dout, dout_strides, 4) &&
+                    aligned16(dq, dq_strides, 4) && aligned16(dk, dk_strides, 4) &&
+                    aligned16(dv, dv_strides, 4);
+    if ((st = launched(mi::launch_attn_bwd_f32(a, 3, al, (hipStream_t)stream),
+                       "attn_bwd_f32")) != MI_OK || !rope)
       return st;
   } else {
     if ((st = mi_attn_bwd_dkdv(dtype, B, H, S, D, causal, scale, q, q_strides, k, k_strides, v,
@@ -447,6 +462,7 @@ mi_status mi_attn_bwd_dkdv(mi_dtype dtype, int B, int H, int S, int D, int causa
   hipStream_t s = (hipStream_t)stream;
   if (al && mi::mfma_supports(dtype, D, S))
     return launched(mi::launch_attn_bwd_dkdv_mfma(dtype, a, s), "attn_bwd_dkdv_mfma");
+  if (dtype == MI_F32) return launched(mi::launch_attn_bwd_f32(a, 1, al, s), "attn_bwd_dkdv_f32");
   return launched(mi::launch_attn_bwd_dkdv_valu(dtype, a, s), "attn_bwd_dkdv_valu");
 }
 
@@ -473,6 +489,7 @@ mi_status mi_attn_bwd_dq(mi_dtype dtype, int B, int H, int S, int D, int causal,
   hipStream_t s = (hipStream_t)stream;
   if (al && mi::mfma_supports(dtype, D, S))
     return launched(mi::launch_attn_bwd_dq_mfma(dtype, a, s), "attn_bwd_dq_mfma");
+  if (dtype == MI_F32) return launched(mi::launch_attn_bwd_f32(a, 2, al, s), "attn_bwd_dq_f32");
   return launched(mi::launch_attn_bwd_dq_valu(dtype, a, s), "attn_bwd_dq_valu");
 }
 

@@ -43,10 +43,18 @@ hipError_t launch_attn_bwd_dkdv_mfma(int dtype, const AttnArgs& a, hipStream_t s
 // dK/dV and dQ in one launch (same results as the two launches above).
 hipError_t launch_attn_bwd_mfma(int dtype, const AttnArgs& a, hipStream_t st);
 hipError_t launch_attn_bwd_dq_mfma(int dtype, const AttnArgs& a, hipStream_t st);
+// fp32 tensors; `vec`: every row 16-byte aligned.  kinds: 1 dK/dV, 2 dQ, 3 both.
+hipError_t launch_attn_fwd_f32(const AttnArgs& a, bool vec, hipStream_t st);
+hipError_t launch_attn_bwd_f32(const AttnArgs& a, int kinds, bool vec, hipStream_t st);
+// 16-bit tensors whose rows are not 16-byte aligned.
 hipError_t launch_attn_fwd_valu(int dtype, const AttnArgs& a, hipStream_t st);
 hipError_t launch_attn_bwd_dkdv_valu(int dtype, const AttnArgs& a, hipStream_t st);
 hipError_t launch_attn_bwd_dq_valu(int dtype, const AttnArgs& a, hipStream_t st);
 hipError_t launch_attn_delta(int dtype, const AttnArgs& a, hipStream_t st);
+
+// Compute units of the device `st` launches on (cached per device), 0 when
+// unknown or not a multiple of the 8 XCDs.
+int cu_count(hipStream_t st);
 
 // Which D values each family is instantiated for.
 bool mfma_supports(int dtype, int D, int S);

@@ -22,8 +22,10 @@
  *   - dtypes: MI_F32, MI_F16, MI_BF16.  Attention runs on bf16/f16 MFMA when
  *     every row is 16-byte aligned, for D = 16, 32, 64 or 128 and any S (16
  *     and 32 in the D = 64 kernels' layout, the padding staged as zeros; no
- *     row at or past S is read or written); every other supported case runs
- *     on an exact-fp32 VALU kernel.  Arithmetic is fp32 in all kernels.
+ *     row at or past S is read or written).  fp32 tensors run on the fp32
+ *     matrix cores at the same D and any S and alignment, with no rounding
+ *     below fp32; bf16/f16 rows that are not 16-byte aligned run on an
+ *     exact-fp32 VALU kernel.
  *
  * Errors: a non-zero mi_status; mi_last_error() gives a message for the
  * calling thread.  Arguments are validated before anything is launched.
