@@ -130,6 +130,27 @@ def lib():
     return _lib
 
 
+_ops = None
+
+
+def ops():
+    """The native host path (csrc/torch_ops.cpp) bound to lib().  Its functions
+    run a plain call and return its result, or return None for any other, which
+    the Python operators then handle or refuse."""
+    global _ops
+    if _ops is None:
+        handle = lib()
+        try:
+            from . import _torch_ops
+        except ImportError as e:
+            raise ImportError("_torch_ops.so is missing or does not load: build it as libmi_attn.so "
+                              f"is built ({e})") from e
+        _torch_ops.bind({n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value
+                         for n in EXPORTED}, MiError)
+        _ops = _torch_ops
+    return _ops
+
+
 def _check(status: int, what: str):
     if status != MI_OK:
         l = lib()

@@ -94,4 +94,5 @@ def attention_block(qkv, cos, sin, heads: int, causal: bool = True):
     """``O = attention(RoPE(q), RoPE(k), v)`` as ``[S, B, H*D]`` from the fused
     qkv projection ``[S, B, 3*H*D]`` (the layout of core/transformer_layer.py:42-61);
     cos/sin are the ``[>= S, D/2]`` tables of ``RotaryEmbedding``."""
-    return AttentionBlock.apply(qkv, cos, sin, heads, causal)
+    o = _lib.ops().attention_block(qkv, cos, sin, heads, causal)
+    return AttentionBlock.apply(qkv, cos, sin, heads, causal) if o is None else o

@@ -68,4 +68,7 @@ _VocabParallelCrossEntropy = VocabParallelCrossEntropy
 
 def vocab_parallel_cross_entropy(logits, target, inplace_backward: bool = False):
     """Per-token loss ``[...]`` of logits ``[..., V]`` against integer targets ``[...]``."""
-    return VocabParallelCrossEntropy.apply(logits, target, inplace_backward)
+    loss = None if inplace_backward else _lib.ops().xent(logits, target)
+    if loss is None:
+        return VocabParallelCrossEntropy.apply(logits, target, inplace_backward)
+    return loss

@@ -78,11 +78,15 @@ class FlashAttn(torch.autograd.Function):
 
 def apply_flash_attn(q, k, v, causal_mask=True):
     """API of core/myFlashAttn.py:1321-1322."""
-    return FlashAttn.apply(q, k, v, causal_mask)
+    o = _lib.ops().flash_attn(q, k, v, causal_mask)
+    return FlashAttn.apply(q, k, v, causal_mask) if o is None else o
 
 
 def flash_attn_forward(q, k, v, causal_mask=True):
     """Forward only, without autograd: returns ``(O, M)`` (M = fp32 logsumexp)."""
+    out = _lib.ops().flash_attn_forward(q, k, v, causal_mask)
+    if out is not None:
+        return out
     B, H, S, D = q.shape
     if not (q.shape == k.shape == v.shape):
         raise AssertionError("Q, K, V must have the same shape")

@@ -45,6 +45,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import _lib
 from ..attention_block import attention_block
 from ..cross_entropy import vocab_parallel_cross_entropy
 from ..mlp import swiglu
@@ -92,7 +93,8 @@ class _LinearGradInto(torch.autograd.Function):
 
 
 def _linear_into_grad(x, w):
-    return _LinearGradInto.apply(x, w)
+    y = _lib.ops().linear_into_grad(x, w) if x.is_cuda else None
+    return _LinearGradInto.apply(x, w) if y is None else y
 
 
 @dataclasses.dataclass

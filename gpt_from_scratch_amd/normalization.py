@@ -95,7 +95,8 @@ class FusedRMSNorm(torch.autograd.Function):
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6,
              grad_into: bool = False) -> torch.Tensor:
-    return FusedRMSNorm.apply(x, weight, eps, grad_into)
+    y = _lib.ops().rms_norm(x, weight, eps, grad_into)
+    return FusedRMSNorm.apply(x, weight, eps, grad_into) if y is None else y
 
 
 def _norm_weight(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -168,7 +169,8 @@ def add_rms_norm(x: torch.Tensor, res: torch.Tensor, weight: torch.Tensor, eps: 
                  grad_into: bool = False):
     """``s = x + res; return s, RMSNorm(s)`` in one kernel (and one backward).
     `grad_into` as for FusedRMSNorm."""
-    return FusedAddRMSNorm.apply(x, res, weight, eps, grad_into)
+    out = _lib.ops().add_rms_norm(x, res, weight, eps, grad_into)
+    return FusedAddRMSNorm.apply(x, res, weight, eps, grad_into) if out is None else out
 
 
 class RMSNorm(nn.Module):
@@ -183,4 +185,4 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(hidden_size, device=device, dtype=torch.float32))
 
     def forward(self, x):
-        return FusedRMSNorm.apply(x, self.weight, self.eps)
+        return rms_norm(x, self.weight, self.eps)

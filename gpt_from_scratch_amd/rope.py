@@ -84,9 +84,11 @@ class RoPEQK(torch.autograd.Function):
 
 def apply_rope(x, cos, sin):
     """API of core/rope_triton.py:144-145."""
-    return RoPE.apply(x, cos, sin)
+    out = _lib.ops().rope(x, cos, sin)
+    return RoPE.apply(x, cos, sin) if out is None else out
 
 
 def apply_rope_qk(q, k, cos, sin):
     """API of core/rope_triton.py:147-148 (one launch for both tensors)."""
-    return RoPEQK.apply(q, k, cos, sin)
+    out = _lib.ops().rope_qk(q, k, cos, sin)
+    return RoPEQK.apply(q, k, cos, sin) if out is None else out
