@@ -348,8 +348,9 @@ __device__ __forceinline__ void store_block_rows_rope_t(const f32x16 (&acc)[D / 
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         float re, ro;
-        rope_rotate(E::to_f32((uint16_t)(v[k] & 0xffffu)), E::to_f32((uint16_t)(v[k] >> 16)),
-                    Tab4<TDT>::get(cs[i], k), Tab4<TDT>::get(sn[i], k), true, re, ro);
+        rope_rotate<std::is_same<E, F16>::value>(
+            E::to_f32((uint16_t)(v[k] & 0xffffu)), E::to_f32((uint16_t)(v[k] >> 16)),
+            Tab4<TDT>::get(cs[i], k), Tab4<TDT>::get(sn[i], k), true, re, ro);
         o[k] = E::pack2(re, ro);
       }
       if (!TAIL || r < nrows) __builtin_nontemporal_store(o, (u32x4*)(grow + (int64_t)r * ss + 8 * c));

@@ -93,6 +93,11 @@ __device__ __forceinline__ uint16_t f32_to_f16(float x) {
 // (RoPE itself, and the attention backward's dQ/dK stores) rounds the same:
 //   forward: (e, o) -> (e c - o s, e s + o c)
 //   inverse: (e, o) -> (e c + o s, o c - e s)
+// F16OUT: the results are rounded to fp16 next.  The compiler may fuse that
+// rounding with the last multiply-add (v_fma_mixlo_f16, one rounding instead of
+// two), here in one kernel and there not in another, and a rare element would
+// differ; the empty asm keeps the fp32 values apart from their rounding.
+template <bool F16OUT>
 __device__ __forceinline__ void rope_rotate(float e, float o, float c, float s, bool inverse,
                                             float& re, float& ro) {
   if (inverse) {
@@ -102,6 +107,7 @@ __device__ __forceinline__ void rope_rotate(float e, float o, float c, float s, 
     re = __builtin_fmaf(e, c, -(o * s));
     ro = __builtin_fmaf(e, s, o * c);
   }
+  if constexpr (F16OUT) asm("" : "+v"(re), "+v"(ro));
 }
 
 // Storage-type traits for kernels that are generic over fp32 / f16 / bf16.

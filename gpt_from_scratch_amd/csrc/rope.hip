@@ -134,7 +134,7 @@ __global__ __launch_bounds__(ROPE_T) void rope_vec_kernel(RopeArgs a, RopeDivs d
           o = F16::to_f32((uint16_t)(x[u][t][p] >> 16));
         }
         float re, ro;
-        rope_rotate(e, o, cs[u][p], sn[u][p], a.inverse != 0, re, ro);
+        rope_rotate<XDT == 1>(e, o, cs[u][p], sn[u][p], a.inverse != 0, re, ro);
         if constexpr (XDT == 0) {
           y[2 * p] = __float_as_uint(re);
           y[2 * p + 1] = __float_as_uint(ro);
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(256) void rope_pair_kernel(RopeArgs a, RopeDivs dv,
   const float cs = ldx<TDT>(a.cos_tab, s * a.cs_s + (int64_t)i * a.cs_i);
   const float sn = ldx<TDT>(a.sin_tab, s * a.ss_s + (int64_t)i * a.ss_i);
   float re, ro;
-  rope_rotate(e, o, cs, sn, a.inverse != 0, re, ro);
+  rope_rotate<XDT == 1>(e, o, cs, sn, a.inverse != 0, re, ro);
   Store<XDT>::st(out, (int64_t)(2 * i) * T.os_d, re);
   Store<XDT>::st(out, (int64_t)(2 * i + 1) * T.os_d, ro);
 }
