@@ -115,9 +115,14 @@ __device__ __forceinline__ constexpr float kProbLimit() {
 // loads are guarded, the tile descriptors end at row S), keys at or past S
 // are masked in the last key tile, which takes the masked step, and rows at
 // or past S are not stored.
-template <typename E, int D, bool CAUSAL, int DP = D, bool RAG = false>
+// KS = 2: a wave takes one 32-key block of each tile instead of both, two waves
+// share 32 query rows, and their O, max and sum are merged at the end; a
+// workgroup owns 64 query rows (see key_split for when, and why).
+template <typename E, int D, bool CAUSAL, int DP = D, bool RAG = false, int KS = 1>
 __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_kernel(AttnArgs a, int n_qtiles, int n_cu) {
   using C = FwdCfg<D>;
+  constexpr int BQ = C::BQ / KS;  // query rows per workgroup
+  constexpr int NB = 2 / KS;      // 32-key blocks of a tile per wave
   static_assert(DP == D || (D == 64 && (DP == 16 || DP == 32)), "head dim");
   constexpr int KSP = DP / 16;         // k-steps of K Q^T over the valid columns
   constexpr int DBP = (DP + 31) / 32;  // O^T blocks holding valid columns
@@ -154,8 +159,9 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
   const uint16_t* vp = (const uint16_t*)a.v.ptr + b * a.v.sb + h * a.v.sh;
   uint16_t* op = (uint16_t*)a.o.ptr + b * a.o.sb + h * a.o.sh;
 
-  const int q0 = qt * C::BQ;
-  const int qw = q0 + 32 * wave;       // first query row of this wave (SGPR)
+  const int q0 = qt * BQ;
+  const int slice = KS == 1 ? 0 : wave & 1;
+  const int qw = q0 + 32 * (KS == 1 ? wave : wave >> 1);  // first query row of this wave (SGPR)
   const bool wave_valid = qw < S;      // without RAG, 32-row blocks are all-or-nothing
   const int qrow = qw + l32;
 
@@ -166,7 +172,7 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
                  ? *(const u32x4*)(qp + (int64_t)qrow * a.q.ss + 16 * ks + 8 * g)
                  : u32x4{0, 0, 0, 0};
 
-  const int kv_end = CAUSAL ? min(q0 + C::BQ, S) : S;
+  const int kv_end = CAUSAL ? min(q0 + BQ, S) : S;
   const int nkv = RAG ? (kv_end + C::BKV - 1) / C::BKV : kv_end / C::BKV;
   // first tile that may need a mask (RAG: the last one holds keys past S)
   const int jdiag = CAUSAL ? q0 / C::BKV : (RAG ? nkv - 1 : nkv);
@@ -207,12 +213,13 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
   // one "buffer + offset" register per buffer out of the step loop.
   int kro[C::KS], vro[C::DB];
 #pragma unroll
-  for (int ks = 0; ks < C::KS; ++ks) kro[ks] = 2 * (l32 * D + (((2 * ks + g) ^ swz_k<D>(l32)) << 3));
+  for (int ks = 0; ks < C::KS; ++ks)
+    kro[ks] = 2 * ((l32 + 32 * slice) * D + (((2 * ks + g) ^ swz_k<D>(l32)) << 3));
 #pragma unroll
   for (int db = 0; db < C::DB; ++db) {
     const int r = 4 * g + ((lane & 15) >> 2);
     const int ch = 4 * db + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-    vro[db] = 2 * (r * D + ((ch ^ swz_v<D>(r)) << 3) + 4 * (lane & 1));
+    vro[db] = 2 * ((r + 32 * slice) * D + ((ch ^ swz_v<D>(r)) << 3) + 4 * (lane & 1));
   }
 
   // ---- per-wave compute pieces ----
@@ -223,31 +230,32 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
   float l_run = 0.f;        // running sum over this lane's half of the keys
   const float c = a.scale_log2;
 
-  // S^T for one key tile (two 32-key blocks).
-  auto qk = [&](const uint16_t* kt, f32x16(&s)[2]) __attribute__((always_inline)) {
+  // S^T for the wave's 32-key blocks of one key tile (kv0: its first block's
+  // first key, here and below).
+  auto qk = [&](const uint16_t* kt, f32x16(&s)[NB]) __attribute__((always_inline)) {
 #pragma unroll
     for (int ks = 0; ks < KSP; ++ks) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
+      for (int kb = 0; kb < NB; ++kb) {
         const u32x4 kf = *(const u32x4*)((const char*)kt + 64 * kb * D + kro[ks]);
         s[kb] = E::mfma(kf, qf[ks], ks == 0 ? f32x16{} : s[kb]);
       }
     }
   };
   // Triangle mask of a diagonal tile (key tile starting at kv0).
-  auto mask = [&](f32x16(&s)[2], int kv0) __attribute__((always_inline)) {
+  auto mask = [&](f32x16(&s)[NB], int kv0) __attribute__((always_inline)) {
     const int rel = qrow - kv0 - 4 * g;  // visible iff (kv - kv0 - 4g) <= rel
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if (32 * kb + 8 * (r >> 2) + (r & 3) > rel) s[kb][r] = -INFINITY;
   };
   // RAG: keys at or past S of the tile starting at kv0 masked.
-  auto mask_tail = [&](f32x16(&s)[2], int kv0) __attribute__((always_inline)) {
+  auto mask_tail = [&](f32x16(&s)[NB], int kv0) __attribute__((always_inline)) {
     const int lim = S - kv0 - 4 * g;  // visible iff (kv - kv0 - 4g) < lim
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if (32 * kb + 8 * (r >> 2) + (r & 3) >= lim) s[kb][r] = -INFINITY;
@@ -256,10 +264,10 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
   // their sum.  D = 64 sums the packed (rounded) values, the ones P V
   // multiplies, with one v_dot2 per pair; D = 128 (where that measured ~1%
   // slower) sums the fp32 values.
-  auto probs = [&](f32x16(&s)[2], u32x4(&pb)[2][2], float mref) __attribute__((always_inline)) {
+  auto probs = [&](f32x16(&s)[NB], u32x4(&pb)[NB][2], float mref) __attribute__((always_inline)) {
     float ps[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+    for (int kb = 0; kb < NB; ++kb) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         s[kb][r] = fast_exp2(__builtin_fmaf(s[kb][r], c, -mref));
@@ -279,12 +287,12 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
   // rescaled) when that exceeds it by more than kRescaleSlack; otherwise the
   // probabilities stay against the stale max, <= 2^8, and exact (O and l share
   // the reference point).
-  auto to_max = [&](f32x16(&s)[2]) __attribute__((always_inline)) {
+  auto to_max = [&](f32x16(&s)[NB]) __attribute__((always_inline)) {
     // NaN-propagating maximum: v_maximum3_f32 chains without input
     // canonicalisation (2 scores per instruction).
     float mx = vmax(s[0][0], s[0][1]);
 #pragma unroll
-    for (int i = 2; i < 32; i += 2) mx = vmax(vmax(mx, s[i >> 4][i & 15]), s[i >> 4][(i & 15) + 1]);
+    for (int i = 2; i < 16 * NB; i += 2) mx = vmax(vmax(mx, s[i >> 4][i & 15]), s[i >> 4][(i & 15) + 1]);
     mx = max_halves(mx) * c;
     if (__any(mx > m_run + kRescaleSlack)) {
       const float m_new = fmaxf(m_run, mx);
@@ -296,9 +304,9 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
     }
   };
   // O^T += V^T P^T.
-  auto pv = [&](const uint16_t* vt, const u32x4(&pb)[2][2]) __attribute__((always_inline)) {
+  auto pv = [&](const uint16_t* vt, const u32x4(&pb)[NB][2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
@@ -330,14 +338,17 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
       dma(vp, a.v.ss, vdo, j + 1, I ? V0 : V1);
     }
     const int kv0 = j * C::BKV;
-    if (wave_valid && (!MASKED || !CAUSAL || kv0 <= qw + 31)) {
-      const bool msk = MASKED && CAUSAL && kv0 + C::BKV - 1 > qw;
-      const bool tmsk = RAG && MASKED && kv0 + C::BKV > S;
-      f32x16 s[2];
+    // first key of the wave's part of the tile; with KS = 2 that part may lie
+    // past the last key
+    const int kw0 = kv0 + 32 * slice;
+    if (wave_valid && (!MASKED || !CAUSAL || kw0 <= qw + 31) && (KS == 1 || !RAG || kw0 < S)) {
+      const bool msk = MASKED && CAUSAL && kw0 + 32 * NB - 1 > qw;
+      const bool tmsk = RAG && MASKED && kw0 + 32 * NB > S;
+      f32x16 s[NB];
       qk(kt, s);
-      if (msk) mask(s, kv0);
-      if (tmsk) mask_tail(s, kv0);
-      u32x4 pb[2][2];
+      if (msk) mask(s, kw0);
+      if (tmsk) mask_tail(s, kw0);
+      u32x4 pb[NB][2];
       // D = 64: probabilities against the running reference m_run without
       // this tile's max, exact as long as their sum stays within kProbLimit
       // (O and l share the reference).  The first tile (no reference yet) and
@@ -345,19 +356,22 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
       // recompute S from the staged K tile and take the exact step.  D = 128
       // takes the exact step every time (the skip's extra code spills there).
       float psum = 0.f;
+      // (KS = 2: a wave's part of the tiles so far may have held -inf scores
+      // alone; it has no reference yet, and takes P = 0 for them)
       bool exact = D != 64 || j == 0;
+      if constexpr (KS > 1) exact = exact || __any(m_run == -INFINITY);
       if (!exact) {
         psum = probs(s, pb, m_run);
         if (__any(!(psum <= kProbLimit<E>()))) {
           exact = true;
           qk(kt, s);
-          if (msk) mask(s, kv0);
-          if (tmsk) mask_tail(s, kv0);
+          if (msk) mask(s, kw0);
+          if (tmsk) mask_tail(s, kw0);
         }
       }
       if (exact) {
         to_max(s);
-        psum = probs(s, pb, m_run);
+        psum = probs(s, pb, KS > 1 && m_run == -INFINITY ? 0.f : m_run);
       }
       l_run += psum;
       pv(vt, pb);
@@ -379,29 +393,89 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
   }
   if (j < nkv) step(j, std::true_type{}, I0_{});
 
-  if (!wave_valid) return;
-  const float l_tot = sum_halves(l_run);
+  float l_tot = sum_halves(l_run);
   // Every buffer is idle after the last step's barrier: wave w stages its O
   // rows through buffer w.
   uint16_t* stage = wave == 0 ? K0 : wave == 1 ? K1 : wave == 2 ? V0 : V1;
+  if constexpr (KS > 1) {
+    // The second wave of a pair hands over its O (through K0 / K1, the
+    // accumulators as they lie), reference and sum; the first takes both to
+    // the larger reference.
+    __shared__ float ml[2][2][64];
+    f32x4* const part = (f32x4*)(wave < 2 ? K0 : K1);
+    float(&pml)[2][64] = ml[wave >> 1];
+    if (slice == 1) {
+#pragma unroll
+      for (int db = 0; db < DBP; ++db)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj)
+          part[(4 * db + jj) * 64 + lane] = f32x4{acc[db][4 * jj], acc[db][4 * jj + 1],
+                                                  acc[db][4 * jj + 2], acc[db][4 * jj + 3]};
+      pml[0][lane] = m_run;
+      pml[1][lane] = l_tot;
+    }
+    __syncthreads();
+    if (slice == 1) return;
+    const float m1 = pml[0][lane], mt = fmaxf(m_run, m1);
+    const float f0 = fast_exp2(m_run - mt), f1 = fast_exp2(m1 - mt);
+    m_run = mt;
+    l_tot = l_tot * f0 + pml[1][lane] * f1;
+#pragma unroll
+    for (int db = 0; db < DBP; ++db)
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        const f32x4 x = part[(4 * db + jj) * 64 + lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[db][4 * jj + i] = __builtin_fmaf(acc[db][4 * jj + i], f0, x[i] * f1);
+      }
+    stage = wave == 0 ? V0 : V1;
+  }
+  if (!wave_valid) return;
   store_block_rows<E, D, DP>(acc, 1.f / l_tot, stage, op + (int64_t)qw * a.o.ss, a.o.ss,
                              RAG ? min(32, S - qw) : 32);
   if (g == 0 && (!RAG || qrow < S)) a.lse[(int64_t)bh * S + qrow] = (m_run + fast_log2(l_tot)) * kLn2;
 }
 
-template <typename E, int D, int DP = D, bool RAG = false>
-hipError_t launch_fwd_d(const AttnArgs& a, hipStream_t st) {
-  const int n_qtiles = (a.S + FwdCfg<D>::BQ - 1) / FwdCfg<D>::BQ;
+// Whether two waves share a query row's keys.  A workgroup is a serial chain of
+// steps (scores, softmax, P V of one key tile), and while waves are few nothing
+// hides its latency: splitting each tile between two waves shortens the step
+// and doubles the workgroups.  Worth it until the chip is full: n = 128-row
+// tiles of all heads against 256 CUs, us whole / split:
+//   causal D = 64     96: 13.9 / 10.0 (B1 H12 S1024)   128: 43.0 / 27.8 (B1 H4 S4096)
+//                    384: 14.9 / 12.3 (B4 H12 S1024)   480: 16.5 / 14.6 (B5 H12 S1024)
+//                    576: 17.1 / 17.1                  768: 19.7 / 22.2 (B8 H12 S1024)
+//   causal D = 128   128: 12.8 / 10.4 (B1 H32 S512)    256: 68.5 / 53.1 (B1 H8 S4096)
+//                    512: 43.4 / 46.3 (B2 H16 S2048)
+//   not causal        96: 13.9 / 10.6 (B1 H12 S1000)   128: 12.0 / 10.0 (D = 128)
+//                    192: 14.0 / 13.6                  256: 21.8 / 23.8 (D = 128)
+// (without the mask all workgroups are equally long: past one per CU the split
+// ones share CUs unevenly.)
+bool key_split(const AttnArgs& a) {
+  const int64_t n = (int64_t)((a.S + 127) / 128) * a.B * a.H;
+  return n <= (!a.causal ? 128 : a.D == 128 ? 256 : 512);
+}
+
+template <typename E, int D, int DP, bool RAG, int KS>
+hipError_t launch_fwd_k(const AttnArgs& a, hipStream_t st) {
+  constexpr int BQ = FwdCfg<D>::BQ / KS;
+  const int n_qtiles = (a.S + BQ - 1) / BQ;
   int n_cu = cu_count(st);
   if (n_cu == 0) n_cu = 1 << 30;  // one round: no reversal
   dim3 grid(n_qtiles * a.B * a.H), block(FwdCfg<D>::NT);
   if (a.causal)
-    hipLaunchKernelGGL((attn_fwd_mfma_kernel<E, D, true, DP, RAG>), grid, block, 0, st, a,
+    hipLaunchKernelGGL((attn_fwd_mfma_kernel<E, D, true, DP, RAG, KS>), grid, block, 0, st, a,
                        n_qtiles, n_cu);
   else
-    hipLaunchKernelGGL((attn_fwd_mfma_kernel<E, D, false, DP, RAG>), grid, block, 0, st, a,
+    hipLaunchKernelGGL((attn_fwd_mfma_kernel<E, D, false, DP, RAG, KS>), grid, block, 0, st, a,
                        n_qtiles, n_cu);
   return hipGetLastError();
+}
+
+template <typename E, int D, int DP = D, bool RAG = false>
+hipError_t launch_fwd_d(const AttnArgs& a, hipStream_t st) {
+  return key_split(a) ? launch_fwd_k<E, D, DP, RAG, 2>(a, st)
+                      : launch_fwd_k<E, D, DP, RAG, 1>(a, st);
 }
 
 template <typename E>

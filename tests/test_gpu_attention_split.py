@@ -1,0 +1,92 @@
+"""The attention kernels' choices by grid size, each against the fp32 oracle.
+
+A small grid has two waves share a row's keys (forward) or an item's tiles
+(backward, head dims 16 to 64), and head dim 128 runs both backward kinds in
+one launch; a large grid does neither.  The head counts below lie on both
+sides of each line (128-row tiles of all heads: 64, 128, 256, 512, 768), at
+lengths at the edges of the 32-row blocks and the 64-row tiles.
+"""
+import pytest
+import torch
+
+from gpu_ref import (MEAN_REL_BF16, assert_close_bf16, budget_ratio, grad_rounding_budget, metrics,
+                     reference, seeded)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    return torch.device("cuda:0")
+
+
+def _run(q, k, v, do, causal):
+    from gpt_from_scratch_amd import flash_attn_backward, flash_attn_forward
+    o, lse = flash_attn_forward(q, k, v, causal)
+    dq, dk, dv, _ = flash_attn_backward(q, k, v, o, lse, do, causal)
+    torch.cuda.synchronize()
+    return o, lse, dq, dk, dv
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("S", [1, 31, 33, 64, 97, 128])
+def test_same_heads_on_every_grid(gpu, S, D, causal):
+    """The first heads of a grid, whatever its size, within the rounding of the
+    oracle; grids on one side of all lines give the same bits."""
+    H = 6
+    q, k, v, do = (seeded((1, H, S, D), 31 * S + D + i).to(gpu) for i in range(4))
+    ref = reference(q, k, v, do, causal, with_backward=False)
+    by_path = {}
+    for n in (H, 64, 65, 128, 130, 256, 258, 512, 514, 768, 770):
+        reps = -(-n // H)
+        big = [t.repeat(1, reps, 1, 1)[:, :n].contiguous() for t in (q, k, v, do)]
+        got = [t[:, :H] for t in _run(*big, causal)]
+        for name, t in (("o", got[0]), ("lse", got[1])):
+            assert_close_bf16(f"{name} n={n}", t, ref[name])
+        want, budget = grad_rounding_budget(q, k, v, do, got[0], causal)
+        for name, t in zip(("dq", "dk", "dv"), got[2:]):
+            worst = budget_ratio(t, want[name], budget[name])
+            assert worst <= 1.0, f"{name} n={n}: error reaches {worst:.3f} of the rounding budget"
+            assert metrics(t, want[name])[1] <= MEAN_REL_BF16, (name, n)
+        fwd = n <= (128 if not causal else 256 if D == 128 else 512)
+        bwd = n <= ((768 if causal else 256) if D == 128 else (256 if causal else 64))
+        first = by_path.setdefault((fwd, bwd), got)
+        assert all(torch.equal(a, b) for a, b in zip(first, got)), n
+    assert len(by_path) > 1
+
+
+@pytest.mark.parametrize("S,D", [(320, 64), (1000, 32), (450, 128)])
+def test_long_chains_split_and_whole(gpu, S, D):
+    """Several tiles per row: strided inputs, fp16, both grid sizes."""
+    for dtype in (torch.bfloat16, torch.float16):
+        for H in (3, 1300 // -(-S // 128)):
+            x = [seeded((S, 1, 3, D), 7 + i, dtype=dtype).to(gpu).repeat(1, 1, H // 3 + 1, 1)[:, :, :H]
+                 .permute(1, 2, 0, 3) for i in range(4)]
+            for causal in (True, False):
+                got = [t[:, :3] for t in _run(*x, causal)]
+                q, k, v, do = (t[:, :3] for t in x)
+                ref = reference(q, k, v, do, causal, with_backward=False)
+                assert_close_bf16("o", got[0], ref["o"])
+                assert_close_bf16("lse", got[1], ref["lse"])
+                want, budget = grad_rounding_budget(q, k, v, do, got[0], causal)
+                for name, t in zip(("dq", "dk", "dv"), got[2:]):
+                    assert budget_ratio(t, want[name], budget[name]) <= 1.0, (name, H, causal)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H", [2, 600])
+def test_scores_of_minus_infinity(gpu, D, H):
+    """Keys that score -inf against every query (all of a wave's part of the
+    first tile, and more) have no part in the rows."""
+    S = 128
+    q, k, v = (seeded((1, 2, S, D), 50 + i).to(gpu).repeat(1, H // 2, 1, 1) for i in range(3))
+    q[..., 0], k[..., 0] = 1.0, 0.0
+    k[:, :, 32:64, 0] = -float("inf")
+    k[:, :, 96:, 0] = -float("inf")
+    from gpt_from_scratch_amd import flash_attn_forward
+    o, lse = flash_attn_forward(q, k, v, False)
+    keep = [j for j in range(S) if j < 32 or 64 <= j < 96]
+    z = q[..., 1:].float() @ k[:, :, keep, 1:].float().transpose(-1, -2).contiguous() / D ** 0.5
+    assert_close_bf16("o", o, z.softmax(-1) @ v[:, :, keep].float())
+    assert_close_bf16("lse", lse, z.logsumexp(-1))
