@@ -226,8 +226,9 @@ struct LdsOffsets {
   }
 };
 
+// `slice`: the 32-row block they start at (the swizzles repeat every 16 rows).
 template <int D, bool SW16 = false>
-__device__ __forceinline__ LdsOffsets<D, SW16> lds_offsets(int lane) {
+__device__ __forceinline__ LdsOffsets<D, SW16> lds_offsets(int lane, int slice = 0) {
   const int l32 = lane & 31;
   const int g = lane >> 5;
   LdsOffsets<D, SW16> o;
@@ -251,6 +252,15 @@ __device__ __forceinline__ LdsOffsets<D, SW16> lds_offsets(int lane) {
       // rows r + 8 (< 16): low three bits as row r, bit 3 of the chunk
       // flipped; the +128 / -128 bytes of that flip is tr_hi's immediate
       o.t2h[db] = 2 * ((r + 8) * D + ((ch ^ (bwd_swz<D, SW16>(r + 8) & 7)) << 3) + 4 * (lane & 1));
+  }
+  if constexpr (D == 64) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) o.r4[ks] += 64 * D * slice;
+#pragma unroll
+    for (int db = 0; db < 2; ++db) {
+      o.t2[db] += 64 * D * slice;
+      o.t2h[db] += 64 * D * slice;
+    }
   }
   return o;
 }
@@ -399,6 +409,13 @@ __device__ __forceinline__ uint16_t* wave_stage_buf(const BwdBuf (&bufs)[2], int
   return (wave & 2) ? b1 : b0;
 }
 
+// The same with KS = 2: the t0 buffer of the pair's own rows.
+template <int KS>
+__device__ __forceinline__ uint16_t* stage_buf(const BwdBuf (&bufs)[2], int wave) {
+  if constexpr (KS == 1) return wave_stage_buf(bufs, wave);
+  else return (wave >> 1) ? bufs[1].t0 : bufs[0].t0;
+}
+
 // Where an item's streamed tiles come from: head bases and strides, and this
 // lane's byte offsets inside a tile for its slices (buffer loads, so that
 // advancing a tile is scalar arithmetic).
@@ -416,16 +433,24 @@ __device__ __forceinline__ const uint16_t* head_ptr(const TensorArg& t, int b, i
   return (const uint16_t*)t.ptr + b * t.sb + h * t.sh;
 }
 
-template <int D, bool CAUSAL>
+template <int D, bool CAUSAL, int KS>
 __device__ __forceinline__ int first_row(const BwdItem& it) {
-  return (CAUSAL && it.kind == 0) ? it.tile * BwdCfg<D>::OWN : 0;
+  return (CAUSAL && it.kind == 0) ? it.tile * (BwdCfg<D>::OWN / KS) : 0;
 }
+
+// The 32 own rows of a wave within its item, and the 32-row block of each
+// streamed tile that it takes with KS = 2 (two waves share the own rows and
+// split the tile; D = 64).
+template <int KS>
+__device__ __forceinline__ int own_block(int wave) { return KS == 1 ? wave : wave >> 1; }
+template <int KS>
+__device__ __forceinline__ int tile_slice(int wave) { return KS == 1 ? 0 : wave & 1; }
 
 // SKIP0: leave res.r[0] unloaded (the D = 128 dK/dV kind keeps K in LDS).
 // DP < D: rows of DP columns; the registers of columns past DP are zeros.
 // RAG: the descriptors end at row S (rows past it load as zeros, lse and
 // delta as 0).
-template <int D, bool SKIP0 = false, int DP = D, bool RAG = false>
+template <int D, bool SKIP0 = false, int DP = D, bool RAG = false, int KS = 1>
 __device__ __forceinline__ void load_resident(const AttnArgs& a, const BwdItem& it,
                                               Resident<D>& res) {
   const int lane = threadIdx.x & 63;
@@ -434,7 +459,7 @@ __device__ __forceinline__ void load_resident(const AttnArgs& a, const BwdItem& 
   const int h = it.bh % a.H;
   const TensorArg& t0 = it.kind ? a.q : a.k;
   const TensorArg& t1 = it.kind ? a.dout : a.v;
-  const int w0 = it.tile * BwdCfg<D>::OWN + 32 * wave;  // first row of this wave (SGPR)
+  const int w0 = it.tile * (BwdCfg<D>::OWN / KS) + 32 * own_block<KS>(wave);  // first row of this wave (SGPR)
   if (w0 < a.S) {
     // wave base in the descriptor, lane offset (row l%32, 8 columns) in one VGPR
     const int nr = RAG ? min(32, a.S - w0) : 32;
@@ -529,6 +554,31 @@ __device__ __forceinline__ void dma_stage(const StageSrc<D>& s, int kind, int ro
   }
 }
 
+// KS = 2: the second wave of a pair hands its accumulators (as they lie) to the
+// first through an idle tile buffer, which adds them to its own.
+template <int DBP, int DB>
+__device__ __forceinline__ void hand_over(const f32x16 (&acc)[DB], uint16_t* buf, int slice,
+                                          int lane) {
+  if (!slice) return;
+#pragma unroll
+  for (int db = 0; db < DBP; ++db)
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj)
+      ((f32x4*)buf)[(4 * db + jj) * 64 + lane] = f32x4{acc[db][4 * jj], acc[db][4 * jj + 1],
+                                                       acc[db][4 * jj + 2], acc[db][4 * jj + 3]};
+}
+template <int DBP, int DB>
+__device__ __forceinline__ void take_over(f32x16 (&acc)[DB], const uint16_t* buf, int lane) {
+#pragma unroll
+  for (int db = 0; db < DBP; ++db)
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const f32x4 x = ((const f32x4*)buf)[(4 * db + jj) * 64 + lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[db][4 * jj + i] += x[i];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // dK / dV item.  Wave w owns keys [kv0 + 32w, +32).  S = Q K^T and
 // dP = dO V^T are computed with keys along the lane index, so P and dS leave
@@ -541,10 +591,13 @@ __device__ __forceinline__ void dma_stage(const StageSrc<D>& s, int kind, int ro
 // accumulators together need ~290 VGPRs, and holding all of them spilled
 // ~390 bytes per lane.  The region then stages the wave's dK and dV stores.
 // ---------------------------------------------------------------------------
-template <typename E, int D, bool CAUSAL, bool ROPE, int DP, bool RAG>
+template <typename E, int D, bool CAUSAL, bool ROPE, int DP, bool RAG, int KS>
 __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
                                           const BwdBuf (&bufs)[2]) {
   using C = BwdCfg<D>;
+  static_assert(KS == 1 || D == 64, "two waves split 64-row tiles");
+  constexpr int OWN = C::OWN / KS;     // own rows of the item
+  constexpr int TB = C::TB / KS;       // 32-row blocks of a tile per wave
   constexpr int KSP = DP / 16;         // k-steps over the valid columns
   constexpr int DBP = (DP + 31) / 32;  // accumulator blocks holding valid columns
   constexpr bool PREFETCH = D == 64;  // operands a block ahead (D = 128 has no registers for it)
@@ -554,22 +607,23 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
   const int g = lane >> 5;
   const int S = a.S;
 
-  const int kv0 = it.tile * C::OWN;
-  const int kw = kv0 + 32 * wave;
+  const int kv0 = it.tile * OWN;
+  const int kw = kv0 + 32 * own_block<KS>(wave);
+  const int slice = tile_slice<KS>(wave);
   const bool wave_valid = kw < S;
   const int b = it.bh / a.H;
   const int h = it.bh % a.H;
   constexpr bool K_IN_LDS = (D == 128);
-  __shared__ __attribute__((aligned(16))) uint16_t k_lds[K_IN_LDS ? C::OWN * D : 8];
+  __shared__ __attribute__((aligned(16))) uint16_t k_lds[K_IN_LDS ? OWN * D : 8];
   uint16_t* const kw_lds = k_lds + (K_IN_LDS ? wave * 32 * D : 0);
 
   // per-lane LDS byte offsets: 16-byte row reads (row l32, chunk 2ks + g) and
   // transposing reads (row 4g + (lane%16)/4, column 32db + 16((lane/16)%2) + 4(lane%4)),
   // and the lane's part of the lse / delta reads (query rows 4g + i of each group of 8)
-  LdsOffsets<D> lo = lds_offsets<D>(lane);
-  int slo = 16 * g;
+  LdsOffsets<D> lo = lds_offsets<D>(lane, slice);
+  int slo = 16 * g + 128 * slice;
 
-  const int q_begin = first_row<D, CAUSAL>(it);
+  const int q_begin = first_row<D, CAUSAL, KS>(it);
   const int nq = RAG ? (S - q_begin + C::TILE - 1) / C::TILE : (S - q_begin) / C::TILE;
   const StageSrc<D> src = stage_src<D, false, DP>(a, it);
 
@@ -599,7 +653,7 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
     }
   }
   Resident<D> res;
-  load_resident<D, K_IN_LDS, DP, RAG>(a, it, res);
+  load_resident<D, K_IN_LDS, DP, RAG, KS>(a, it, res);
   const u32x4(&kf)[C::KS] = res.r[0];
   const u32x4(&vn)[C::KS] = res.r[1];  // -V
   __syncthreads();
@@ -614,8 +668,9 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
     constexpr bool LAST = decltype(last_tag)::value;
     constexpr int P = decltype(parity)::value;
     const int q0 = q_begin + j * C::TILE;
-    // (at D = 128 the last step is not peeled: a uniform branch skips its load)
-    if (!LAST && (D == 64 || j + 1 < nq))
+    // (at D = 128 and with KS = 2 the last step is not peeled: a uniform branch
+    // skips its load)
+    if (!LAST && ((D == 64 && KS == 1) || j + 1 < nq))
       dma_stage<D, DP, RAG>(src, 0, q0 + C::TILE, bufs[P ^ 1], S);
 
     lo.refresh();
@@ -624,15 +679,15 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
       const uint16_t* Qs = bufs[P].t0;
       const uint16_t* dOs = bufs[P].t1;
       const float* sl = bufs[P].sl;
-      u32x4 pb[C::TB][2], sb[C::TB][2];
-      bool live[C::TB];
+      u32x4 pb[TB][2], sb[TB][2];
+      bool live[TB];
       // Each block's A operands and delta rows are requested before its first
       // product: block 0's at the top of the step, block 1's right after
       // block 0's products are issued (one LDS round trip per block instead
       // of one per product).  The scheduling barriers keep the compiler from
       // sinking the reads back next to their uses.
       u32x4 qa[KSP], da[KSP];
-      f32x16 sacc[C::TB], dpacc[C::TB];
+      f32x16 sacc[TB], dpacc[TB];
       auto read_ops = [&](int qb) __attribute__((always_inline)) {
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
@@ -651,8 +706,8 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int qb = 0; qb < C::TB; ++qb) {
-        const int qbs = q0 + 32 * qb;
+      for (int qb = 0; qb < TB; ++qb) {
+        const int qbs = q0 + 32 * (slice + qb);
         live[qb] = !MASKED || (qbs + 31 >= kw);
         if constexpr (!PREFETCH) read_ops(qb);
         if (live[qb]) {
@@ -668,16 +723,16 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
           for (int ks = 0; ks < KSP; ++ks) dpacc[qb] = E::mfma(da[ks], vn[ks], dpacc[qb]);
         }
         if constexpr (PREFETCH) {
-          if (qb + 1 < C::TB) {
+          if (qb + 1 < TB) {
             read_ops(qb + 1);
             __builtin_amdgcn_sched_barrier(0);
           }
         }
       }
 #pragma unroll
-      for (int qb = 0; qb < C::TB; ++qb) {
+      for (int qb = 0; qb < TB; ++qb) {
         if (!live[qb]) continue;
-        const int qbs = q0 + 32 * qb;
+        const int qbs = q0 + 32 * (slice + qb);
         f32x16& s = sacc[qb];
         f32x16& dp = dpacc[qb];
         const bool diag = MASKED && qbs == kw;
@@ -704,7 +759,7 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
           }
       }
 #pragma unroll
-      for (int qb = 0; qb < C::TB; ++qb) {
+      for (int qb = 0; qb < TB; ++qb) {
         if (!live[qb]) continue;
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
@@ -737,17 +792,21 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
     if (j < j_end) step(j++, masked_tag, std::false_type{}, P0{});
   };
   // nq >= 1 (S > q_begin)
-  if constexpr (D == 128) {
+  if constexpr (KS > 1) {
+    // only the first tile straddles the 64 own keys
+    step(j++, std::integral_constant<bool, CAUSAL>{}, std::false_type{}, P0{});
+    run(nq, std::false_type{});
+  } else if constexpr (D == 128) {
     // Peeled last steps (four more copies of the step) raised the register
     // pressure of the whole item past 256 and spilled; here the loop runs to
     // nq and the step skips the load past the end.
-    if constexpr (CAUSAL) run(min(nq, C::OWN / C::TILE), std::true_type{});
+    if constexpr (CAUSAL) run(min(nq, OWN / C::TILE), std::true_type{});
     run(nq, std::false_type{});
   } else {
-    const int n_diag = CAUSAL ? min(nq - 1, C::OWN / C::TILE) : 0;
+    const int n_diag = CAUSAL ? min(nq - 1, OWN / C::TILE) : 0;
     if constexpr (CAUSAL) run(n_diag, std::true_type{});
     run(nq - 1, std::false_type{});
-    const bool last_masked = CAUSAL && nq - 1 < C::OWN / C::TILE;
+    const bool last_masked = CAUSAL && nq - 1 < OWN / C::TILE;
     if (last_masked) {
       if (j & 1) step(j, std::true_type{}, std::true_type{}, P1{});
       else step(j, std::true_type{}, std::true_type{}, P0{});
@@ -757,6 +816,16 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
     }
   }
 
+  if constexpr (KS > 1) {
+    // tile buffers: dV and dK of the first own rows, then of the second
+    const BwdBuf& mine = own_block<KS>(wave) ? bufs[1] : bufs[0];
+    hand_over<DBP>(dv, mine.t0, slice, lane);
+    hand_over<DBP>(dk, mine.t1, slice, lane);
+    __syncthreads();
+    if (slice) return;
+    take_over<DBP>(dv, mine.t0, lane);
+    take_over<DBP>(dk, mine.t1, lane);
+  }
   if (!wave_valid) return;
   const int nrows = RAG ? min(32, S - kw) : 32;  // keys of this wave below S
   uint16_t* const dk_rows = (uint16_t*)a.dk.ptr + b * a.dk.sb + h * a.dk.sh + (int64_t)kw * a.dk.ss;
@@ -764,7 +833,7 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
   if constexpr (D == 64) {
     // The staging buffers are idle after the last step's barrier: wave w
     // stages its rows (dK, then dV) through tile buffer w.
-    uint16_t* stage = wave_stage_buf(bufs, wave);
+    uint16_t* stage = stage_buf<KS>(bufs, wave);
     // dV first: its accumulators are dead before dK's rotation needs registers
     store_block_rows<E, D, DP>(dv, 1.f, stage, dv_rows, a.dv.ss, nrows);
     if (ROPE && a.rope.cos)
@@ -790,10 +859,13 @@ __device__ __forceinline__ void dkdv_item(const AttnArgs& a, const BwdItem& it,
 // per-lane scalars and dS^T feeds dQ^T = K^T dS^T directly (K^T read
 // transposed from the K tile).
 // ---------------------------------------------------------------------------
-template <typename E, int D, bool CAUSAL, bool ROPE, int DP, bool RAG>
+template <typename E, int D, bool CAUSAL, bool ROPE, int DP, bool RAG, int KS>
 __device__ __forceinline__ void dq_item(const AttnArgs& a, const BwdItem& it,
                                         const BwdBuf (&bufs)[2]) {
   using C = BwdCfg<D>;
+  static_assert(KS == 1 || D == 64, "two waves split 64-row tiles");
+  constexpr int OWN = C::OWN / KS;     // own rows of the item
+  constexpr int TB = C::TB / KS;       // 32-row blocks of a tile per wave
   constexpr int KSP = DP / 16;         // k-steps over the valid columns
   constexpr int DBP = (DP + 31) / 32;  // accumulator blocks holding valid columns
   static_assert(D == 64 || D == 128, "head dim of the item layout");
@@ -804,14 +876,15 @@ __device__ __forceinline__ void dq_item(const AttnArgs& a, const BwdItem& it,
   const int g = lane >> 5;
   const int S = a.S;
 
-  const int q0 = it.tile * C::OWN;
-  const int qw = q0 + 32 * wave;
+  const int q0 = it.tile * OWN;
+  const int qw = q0 + 32 * own_block<KS>(wave);
+  const int slice = tile_slice<KS>(wave);
   const bool wave_valid = qw < S;
 
   // D = 128: the 4-bit swizzle (conflict-free row reads), see bwd_swz
-  LdsOffsets<D, D == 128> lo = lds_offsets<D, D == 128>(lane);
+  LdsOffsets<D, D == 128> lo = lds_offsets<D, D == 128>(lane, slice);
 
-  const int kv_end = CAUSAL ? min(q0 + C::OWN, S) : S;
+  const int kv_end = CAUSAL ? min(q0 + OWN, S) : S;
   const int nkv = RAG ? (kv_end + C::TILE - 1) / C::TILE : kv_end / C::TILE;
   const StageSrc<D> src = stage_src<D, D == 128, DP>(a, it);
 
@@ -823,7 +896,7 @@ __device__ __forceinline__ void dq_item(const AttnArgs& a, const BwdItem& it,
   // First tile's loads before the resident rows (one round trip for both).
   dma_stage<D, DP, RAG>(src, 1, 0, bufs[0], S);
   Resident<D> res;
-  load_resident<D, false, DP, RAG>(a, it, res);
+  load_resident<D, false, DP, RAG, KS>(a, it, res);
   const u32x4(&qf)[C::KS] = res.r[0];
   const u32x4(&df)[C::KS] = res.r[1];
   const float lse2 = res.lse2;
@@ -850,13 +923,13 @@ __device__ __forceinline__ void dq_item(const AttnArgs& a, const BwdItem& it,
     if (wave_valid && (!MASKED || kv0 <= qw + 31)) {
       const uint16_t* Ks = bufs[P].t0;
       const uint16_t* Vs = bufs[P].t1;
-      u32x4 sb[C::TB][2];
-      bool live[C::TB];
+      u32x4 sb[TB][2];
+      bool live[TB];
       // Each block's A operands requested before its first product (block
       // 0's at the top of the step, block 1's once block 0's products are
       // issued), as in the dK/dV item.
       u32x4 ka[KSP], va[KSP];
-      f32x16 sacc[C::TB], dpacc[C::TB];
+      f32x16 sacc[TB], dpacc[TB];
       auto read_ops = [&](int kb) __attribute__((always_inline)) {
 #pragma unroll
         for (int ks = 0; ks < KSP; ++ks) {
@@ -877,8 +950,8 @@ __device__ __forceinline__ void dq_item(const AttnArgs& a, const BwdItem& it,
         for (int ks = 0; ks < KSP; ++ks) va[ks] = *lds_at<u32x4>(Vs, lo.row(ks));
       }
 #pragma unroll
-      for (int kb = 0; kb < C::TB; ++kb) {
-        const int kvb = kv0 + 32 * kb;
+      for (int kb = 0; kb < TB; ++kb) {
+        const int kvb = kv0 + 32 * (slice + kb);
         live[kb] = !MASKED || (kvb <= qw + 31);
         if (live[kb]) {
           sacc[kb] = f32x16{};
@@ -890,16 +963,16 @@ __device__ __forceinline__ void dq_item(const AttnArgs& a, const BwdItem& it,
           for (int ks = 0; ks < KSP; ++ks) dpacc[kb] = E::mfma(va[ks], df[ks], dpacc[kb]);
         }
         if constexpr (PREFETCH) {
-          if (kb + 1 < C::TB) {
+          if (kb + 1 < TB) {
             read_ops(kb + 1);
             __builtin_amdgcn_sched_barrier(0);
           }
         }
       }
 #pragma unroll
-      for (int kb = 0; kb < C::TB; ++kb) {
+      for (int kb = 0; kb < TB; ++kb) {
         if (!live[kb]) continue;
-        const int kvb = kv0 + 32 * kb;
+        const int kvb = kv0 + 32 * (slice + kb);
         f32x16& s = sacc[kb];
         f32x16& dp = dpacc[kb];
         const bool diag = MASKED && kvb == qw;
@@ -920,7 +993,7 @@ __device__ __forceinline__ void dq_item(const AttnArgs& a, const BwdItem& it,
             sb[kb][hh][w] = E::pack2(dp[8 * hh + 2 * w], dp[8 * hh + 2 * w + 1]);
       }
 #pragma unroll
-      for (int kb = 0; kb < C::TB; ++kb) {
+      for (int kb = 0; kb < TB; ++kb) {
         if (!live[kb]) continue;
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
@@ -949,18 +1022,22 @@ __device__ __forceinline__ void dq_item(const AttnArgs& a, const BwdItem& it,
     if (j < j_end) step(j++, masked_tag, std::false_type{}, P0{});
   };
   // nkv >= 1 (kv_end > 0)
-  const int n_main = CAUSAL ? max(0, nkv - C::OWN / C::TILE) : nkv;
+  // Causal: the last OWN / TILE tiles straddle the own queries, the last one
+  // always (with KS = 2 it alone does).
+  const int n_main = CAUSAL ? max(0, nkv - OWN / C::TILE) : nkv;
   run(min(n_main, nkv - 1), std::false_type{});
-  if constexpr (CAUSAL) run(nkv - 1, std::true_type{});
-  const bool last_masked = CAUSAL && nkv - 1 >= n_main;
-  if (last_masked) {
-    if (j & 1) step(j, std::true_type{}, std::true_type{}, P1{});
-    else step(j, std::true_type{}, std::true_type{}, P0{});
-  } else {
-    if (j & 1) step(j, std::false_type{}, std::true_type{}, P1{});
-    else step(j, std::false_type{}, std::true_type{}, P0{});
-  }
+  if constexpr (CAUSAL && OWN > C::TILE) run(nkv - 1, std::true_type{});
+  using LastMasked = std::integral_constant<bool, CAUSAL>;
+  if (j & 1) step(j, LastMasked{}, std::true_type{}, P1{});
+  else step(j, LastMasked{}, std::true_type{}, P0{});
 
+  if constexpr (KS > 1) {
+    uint16_t* const part = stage_buf<KS>(bufs, wave);
+    hand_over<DBP>(acc, part, slice, lane);
+    __syncthreads();
+    if (slice) return;
+    take_over<DBP>(acc, part, lane);
+  }
   if (!wave_valid) return;
   const int b = it.bh / a.H;
   const int h = it.bh % a.H;
@@ -968,17 +1045,17 @@ __device__ __forceinline__ void dq_item(const AttnArgs& a, const BwdItem& it,
       (uint16_t*)a.dq.ptr + b * a.dq.sb + h * a.dq.sh + (int64_t)qw * a.dq.ss;
   const int nrows = RAG ? min(32, S - qw) : 32;  // queries of this wave below S
   if (ROPE && a.rope.cos)
-    store_block_rows_rope<E, D, RAG>(acc, a.scale, wave_stage_buf(bufs, wave), dq_rows, a.dq.ss,
+    store_block_rows_rope<E, D, RAG>(acc, a.scale, stage_buf<KS>(bufs, wave), dq_rows, a.dq.ss,
                                 a.rope, qw, nrows);
   else
-    store_block_rows<E, D, DP>(acc, a.scale, wave_stage_buf(bufs, wave), dq_rows, a.dq.ss,
+    store_block_rows<E, D, DP>(acc, a.scale, stage_buf<KS>(bufs, wave), dq_rows, a.dq.ss,
                                nrows);
 }
 
 // One item per workgroup.  One LDS array per buffer and tensor, so that the
 // compiler can see that a direct load into one buffer never aliases the
 // reads of the other.
-template <typename E, int D, bool CAUSAL, bool ROPE, int DP = D, bool RAG = false>
+template <typename E, int D, bool CAUSAL, bool ROPE, int DP = D, bool RAG = false, int KS = 1>
 __device__ __forceinline__ void run_item(const AttnArgs& a, const BwdItem it) {
   using C = BwdCfg<D>;
   __shared__ __attribute__((aligned(16))) uint16_t A0[C::ELEMS];
@@ -989,9 +1066,9 @@ __device__ __forceinline__ void run_item(const AttnArgs& a, const BwdItem it) {
   __shared__ __attribute__((aligned(16))) float SB[2 * C::TILE];
   const BwdBuf bufs[2] = {{A0, A1, SA}, {B0, B1, SB}};
   if (it.kind)
-    dq_item<E, D, CAUSAL, ROPE, DP, RAG>(a, it, bufs);
+    dq_item<E, D, CAUSAL, ROPE, DP, RAG, KS>(a, it, bufs);
   else
-    dkdv_item<E, D, CAUSAL, ROPE, DP, RAG>(a, it, bufs);
+    dkdv_item<E, D, CAUSAL, ROPE, DP, RAG, KS>(a, it, bufs);
 }
 
 // ROPE (every kernel below): the kernel carries the rotating stores, and dQ
@@ -1039,6 +1116,44 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(AttnArgs a, int n_tile
       a, BwdItem{kind, kind ? n_tiles - 1 - r : r, (int)(blockIdx.x % BH)});
 }
 
+// The same with 64 own rows per item, shared by two waves that split each
+// tile (see tile_split).
+template <typename E, bool CAUSAL, bool ROPE, int DP, bool RAG>
+__global__ __launch_bounds__(256, 2) void attn_bwd_split_kernel(AttnArgs a, int n_tiles,
+                                                                int only_kind) {
+  const int BH = a.B * a.H;
+  const int rank = blockIdx.x / BH;
+  const int kind = only_kind < 0 ? rank & 1 : only_kind;
+  const int r = only_kind < 0 ? rank >> 1 : rank;
+  run_item<E, 64, CAUSAL, ROPE, DP, RAG, 2>(
+      a, BwdItem{kind, kind ? n_tiles - 1 - r : r, (int)(blockIdx.x % BH)});
+}
+
+// 128-row tiles of all heads: the items of one kind, and the measure of how
+// full a launch makes the chip (256 CUs, two workgroups of these kernels each).
+int64_t tiles128(const AttnArgs& a) { return (int64_t)((a.S + 127) / 128) * a.B * a.H; }
+
+// Whether two waves share the own rows of an item (head dims 16 to 64).  An
+// item is a serial chain of steps, and a launch that leaves slots empty lasts
+// as long as its longest one: splitting the tiles makes each step shorter and
+// the items twice as many.  us, whole / split, D = 64, by tiles128:
+//   causal      48: 11.8 / 9.7 (B1 H12 S512)     96: 18.9 / 15.5 (B1 H12 S1024)
+//              128: 61.1 / 50.7 (B1 H4 S4096)   192: 37.0 / 31.8 (B1 H12 S2048)
+//              256: 22.3 / 22.1 (B4 H8 S1024)   384: 30.1 / 30.5 (B4 H12 S1024)
+//   not causal  64: 18.0 / 14.7 (B1 H8 S1024)    96: 18.7 / 20.8 (B1 H12 S1000)
+// (without the mask all items are equally long, and 96 tiles split are 384
+// items: half the CUs get two.)
+bool tile_split(const AttnArgs& a) { return tiles128(a) <= (a.causal ? 256 : 64); }
+
+// Whether D = 128 runs both kinds in one launch.  The kinds alone are faster
+// kernels, but two launches in a row each wait for their own longest items.
+// us, two launches / one, by tiles128:
+//   causal      128: 38.9 / 22.9 (B1 H32 S512)     256: 237 / 180 (B1 H8 S4096)
+//               512: 153 / 119 (B2 H16 S2048)      768: 188 / 180 (B3 H16 S2048)
+//              1024: 436 / 439 (B2 H16 S4096)     2048: 1734 / 1791 (B1 H32 S8192)
+//   not causal  256: 70.7 / 63.2 (B1 H32 S1024)    512: 219 / 239 (B2 H16 S2048)
+bool one_launch(const AttnArgs& a) { return tiles128(a) <= (a.causal ? 768 : 256); }
+
 template <typename E, int D, bool ROPE, bool RAG = false>
 hipError_t launch_dkdv_dr(const AttnArgs& a, hipStream_t st) {
   const int BH = a.B * a.H;
@@ -1073,6 +1188,15 @@ hipError_t launch_dq_dr(const AttnArgs& a, hipStream_t st) {
 template <typename E, int D, bool CAUSAL, int DP = D, bool RAG = false>
 hipError_t launch_both_dc(const AttnArgs& a, int only_kind, hipStream_t st) {
   const int BH = a.B * a.H;
+  if constexpr (D == 64) {
+    if (tile_split(a)) {
+      const int n2 = (a.S + 63) / 64;
+      hipLaunchKernelGGL((attn_bwd_split_kernel<E, CAUSAL, DP == D, DP, RAG>),
+                         dim3((only_kind < 0 ? 2 : 1) * n2 * BH), dim3(256), 0, st, a, n2,
+                         only_kind);
+      return hipGetLastError();
+    }
+  }
   const int n = (a.S + BwdCfg<D>::OWN - 1) / BwdCfg<D>::OWN;
   hipLaunchKernelGGL((attn_bwd_kernel<E, D, CAUSAL, DP == D, DP, RAG>),
                      dim3((only_kind < 0 ? 2 : 1) * n * BH), dim3(256), 0, st, a, n, only_kind);
@@ -1138,15 +1262,15 @@ hipError_t launch_dq_e(const AttnArgs& a, hipStream_t st) {
   return rag ? launch_dq_d<E, 128, true>(a, st) : launch_dq_d<E, 128>(a, st);
 }
 
-// D = 128: two launches.  Both kinds sit at the 256-register limit of two waves
-// per SIMD there, and one combined launch measured 10-15% slower than the two
-// (when the dK/dV kind still held K in registers and spilled).
+// D = 128: one launch or two (one_launch).
 template <typename E>
 hipError_t launch_both_e(const AttnArgs& a, hipStream_t st) {
   if (a.D < 64) return launch_small_d<E>(a, st, -1);
   const bool rag = a.S % 64 != 0;
   if (a.D == 64)
     return rag ? launch_both_d<E, 64, 64, true>(a, st) : launch_both_d<E, 64>(a, st);
+  if (one_launch(a))
+    return rag ? launch_both_d<E, 128, 128, true>(a, st) : launch_both_d<E, 128>(a, st);
   hipError_t e = rag ? launch_dkdv_d<E, 128, true>(a, st) : launch_dkdv_d<E, 128>(a, st);
   if (e != hipSuccess) return e;
   return rag ? launch_dq_d<E, 128, true>(a, st) : launch_dq_d<E, 128>(a, st);
