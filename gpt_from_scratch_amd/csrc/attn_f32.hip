@@ -426,7 +426,7 @@ __device__ __forceinline__ void bwd_item(const AttnArgs& a, int bh, int r0, floa
   // One tile; only masked tiles (the diagonal and the tails) have branches.
   auto step = [&](int row0, auto masked) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked)::value;
-#pragma unroll 1
+#pragma unroll 2
     for (int n = 0; n < NB; ++n) {
       const int blk = slice + KS * n, s0 = row0 + 16 * blk;
       if (MASKED && (s0 >= S || (causal && (DKDV ? s0 + 15 < rw : s0 > rw + 15)))) continue;
