@@ -28,7 +28,8 @@ EXPORTED = ("mi_version", "mi_status_str", "mi_last_error", "mi_attn_fwd", "mi_a
             "mi_rmsnorm_bwd_workspace", "mi_rmsnorm_bwd", "mi_swiglu_fwd", "mi_swiglu_bwd",
             "mi_adamw_workspace", "mi_grad_sumsq", "mi_adamw_step", "mi_attn_bwd_noalloc",
             "mi_rmsnorm_add_fwd", "mi_rmsnorm_add_bwd", "mi_attn_bwd_rope",
-            "mi_rmsnorm_bwd_acc", "mi_rmsnorm_add_bwd_acc", "mi_copy_qk")
+            "mi_rmsnorm_bwd_acc", "mi_rmsnorm_add_bwd_acc", "mi_copy_qk",
+            "mi_wgrad_workspace", "mi_wgrad_suits", "mi_wgrad")
 
 # B*H*S limit of mi_attn_bwd_noalloc (its static workspace array), include/mi_attn.h
 NOALLOC_MAX_ROWS = 1 << 20
@@ -108,6 +109,12 @@ def _declare(lib):
     lib.mi_swiglu_fwd.argtypes = [i, i64, i64, p, i64, p, i64, p]
     lib.mi_swiglu_bwd.restype = i
     lib.mi_swiglu_bwd.argtypes = [i, i64, i64, p, i64, p, i64, p, i64, p]
+    lib.mi_wgrad_workspace.restype = i64
+    lib.mi_wgrad_workspace.argtypes = [i64, i64, i64]
+    lib.mi_wgrad_suits.restype = i
+    lib.mi_wgrad_suits.argtypes = [i64, i64, i64]
+    lib.mi_wgrad.restype = i
+    lib.mi_wgrad.argtypes = [i, i64, i64, i64, p, i64, p, i64, p, i, p, i64, p]
     lib.mi_adamw_workspace.restype = i64
     lib.mi_adamw_workspace.argtypes = []
     lib.mi_grad_sumsq.restype = i
@@ -424,6 +431,34 @@ def swiglu_bwd(gate_up, dout, dgate_up):
     st = lib().mi_swiglu_bwd(dtype_code(gate_up), rows, dout.shape[-1], _ptr(gate_up), gs,
                              _ptr(dout), ds, _ptr(dgate_up), dgs, _stream(gate_up))
     _check(st, "mi_swiglu_bwd")
+
+
+def wgrad(dy, x, dweight=None):
+    """Enqueue the weight gradient dy^T x of a projection (dy [rows, out], x
+    [rows, in]): added to `dweight` [out, in], or into a new tensor.  Returns the
+    gradient, or None (nothing enqueued) where the kernel does not suit and a
+    general GEMM is to be used."""
+    if dy.device.type != "cuda" or x.device != dy.device or dy.dtype != x.dtype \
+            or dy.dtype not in (torch.bfloat16, torch.float16):
+        return None
+    rows, out = dy.shape
+    if not lib().mi_wgrad_suits(rows, out, x.shape[1]):
+        return None
+    for t in (dy, x):
+        if t.stride(1) != 1 or t.stride(0) < t.shape[1] or t.stride(0) >= 1 << 24 \
+                or t.stride(0) % 8 or t.shape[1] % 8 or t.data_ptr() % 16:
+            return None
+    acc = dweight is not None
+    if not acc:
+        dweight = torch.empty(out, x.shape[1], dtype=dy.dtype, device=dy.device)
+    elif dweight.dtype != dy.dtype or dweight.device != dy.device or dweight.data_ptr() % 8:
+        return None
+    n = lib().mi_wgrad_workspace(rows, out, x.shape[1])
+    ws = torch.empty(n, dtype=torch.float32, device=dy.device)
+    st = lib().mi_wgrad(dtype_code(dy), rows, out, x.shape[1], _ptr(dy), dy.stride(0), _ptr(x),
+                        x.stride(0), _ptr(dweight), int(acc), _ptr(ws), n, _stream(dy))
+    _check(st, "mi_wgrad")
+    return dweight
 
 
 def adamw_workspace() -> int:

@@ -956,6 +956,58 @@ mi_status mi_swiglu_bwd(mi_dtype dtype, int64_t rows, int64_t inter, const void*
                   "swiglu_bwd");
 }
 
+int64_t mi_wgrad_workspace(int64_t rows, int64_t out_features, int64_t in_features) {
+  if (rows <= 0 || out_features <= 0 || in_features <= 0) return 0;
+  return mi::wgrad_splits(rows, out_features, in_features) * out_features * in_features;
+}
+
+int mi_wgrad_suits(int64_t rows, int64_t out_features, int64_t in_features) {
+  return rows > 0 && out_features > 0 && in_features > 0 &&
+         mi::wgrad_suits(rows, out_features, in_features);
+}
+
+mi_status mi_wgrad(mi_dtype dtype, int64_t rows, int64_t out_features, int64_t in_features,
+                   const void* dy, int64_t dy_row_stride, const void* x, int64_t x_row_stride,
+                   void* dweight, int accumulate, float* workspace, int64_t workspace_elems,
+                   void* stream) {
+  MI_SOLE_COPY();
+  if (dtype != MI_BF16 && dtype != MI_F16)
+    return fail(MI_ERR_INVALID_ARGUMENT, "dtype %d: bf16 or f16 wanted", dtype);
+  if (rows <= 0 || out_features <= 0 || in_features <= 0 || rows >= (1ll << 31) ||
+      out_features >= (1ll << 24) || in_features >= (1ll << 24))
+    return fail(MI_ERR_INVALID_ARGUMENT, "sizes out of range (rows=%lld out=%lld in=%lld)",
+                (long long)rows, (long long)out_features, (long long)in_features);
+  if (!dy || !x || !dweight || !workspace)
+    return fail(MI_ERR_INVALID_ARGUMENT, "dy / x / dweight / workspace: null pointer");
+  // 16-byte loads of dy and x rows, 8-byte ones of dweight; 64 rows of either
+  // operand within the 31-bit offsets of the buffer loads
+  if (out_features % 8 || in_features % 8 || dy_row_stride % 8 || x_row_stride % 8 ||
+      ((uintptr_t)dy) % 16 || ((uintptr_t)x) % 16 || ((uintptr_t)dweight) % 8 ||
+      ((uintptr_t)workspace) % 16)
+    return fail(MI_ERR_UNSUPPORTED, "rows must be 16-byte aligned and of a multiple of 8 elements");
+  if (dy_row_stride < out_features || x_row_stride < in_features ||
+      dy_row_stride >= (1ll << 24) || x_row_stride >= (1ll << 24))
+    return fail(MI_ERR_INVALID_ARGUMENT, "row strides %lld, %lld out of range",
+                (long long)dy_row_stride, (long long)x_row_stride);
+  const int splits = mi::wgrad_splits(rows, out_features, in_features);
+  if (workspace_elems < splits * out_features * in_features)
+    return fail(MI_ERR_INVALID_ARGUMENT, "workspace: %lld elements, %lld wanted",
+                (long long)workspace_elems, (long long)(splits * out_features * in_features));
+  mi::WgradArgs a = {};
+  a.dy = dy;
+  a.dys = dy_row_stride;
+  a.x = x;
+  a.xs = x_row_stride;
+  a.dw = dweight;
+  a.part = workspace;
+  a.M = (int)rows;
+  a.N = (int)out_features;
+  a.K = (int)in_features;
+  a.splits = splits;
+  a.acc = accumulate ? 1 : 0;
+  return launched(mi::launch_wgrad(dtype, a, (hipStream_t)stream), "wgrad");
+}
+
 int64_t mi_adamw_workspace(void) { return 1 + mi::adam_parts(); }
 
 mi_status mi_grad_sumsq(mi_dtype grad_dtype, int64_t n, const void* grad, float* workspace,

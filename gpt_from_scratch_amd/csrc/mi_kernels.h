@@ -144,6 +144,23 @@ hipError_t launch_swiglu(bool bwd, int dtype, int64_t rows, int64_t inter, const
                          int64_t gu_stride, const void* dh, int64_t dh_stride, void* out,
                          int64_t out_stride, bool vec, hipStream_t st);
 
+// Weight gradient dW[N, K] = dY[M, N]^T X[M, K] (+ dW with acc) of a projection
+// (wgrad.hip): rows of dy and x are dys and xs elements apart, dw is dense, part
+// is an fp32 workspace of splits * N * K elements.
+struct WgradArgs {
+  const void* dy;
+  int64_t dys;
+  const void* x;
+  int64_t xs;
+  void* dw;
+  float* part;
+  int M, N, K, splits, acc;
+  int tn, tk;  // 128 x 128 tiles of dw (set by the launcher)
+};
+int wgrad_splits(int64_t M, int64_t N, int64_t K);
+bool wgrad_suits(int64_t M, int64_t N, int64_t K);
+hipError_t launch_wgrad(int dtype, WgradArgs a, hipStream_t st);
+
 // The optimizer step (model_ops.hip).  Squared gradient norm into out[0] via
 // adam_parts() partial sums; the AdamW step over the flat buffers with
 // hp = {1 - lr*wd, 1 - beta1, beta2, 1 - beta2, lr / (1 - beta1^t),

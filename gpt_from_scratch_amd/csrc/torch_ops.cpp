@@ -46,7 +46,7 @@ using torch::autograd::variable_list;
   X(mi_rope) X(mi_rope_qk) X(mi_xent_fwd) X(mi_xent_bwd) X(mi_rmsnorm_fwd)                 \
   X(mi_rmsnorm_bwd_workspace) X(mi_rmsnorm_bwd) X(mi_rmsnorm_bwd_acc)                      \
   X(mi_rmsnorm_add_fwd) X(mi_rmsnorm_add_bwd) X(mi_rmsnorm_add_bwd_acc) X(mi_swiglu_fwd)   \
-  X(mi_swiglu_bwd)
+  X(mi_swiglu_bwd) X(mi_wgrad_suits) X(mi_wgrad_workspace) X(mi_wgrad)
 
 struct Bound {
 #define X(f) decltype(&::f) f = nullptr;
@@ -556,23 +556,50 @@ struct SwiGLU : torch::autograd::Function<SwiGLU> {
   }
 };
 
+// dy^T x added to g, or in a new tensor (_lib.wgrad); undefined where a general
+// GEMM is to be used.
+Tensor wgrad(const Tensor& dy, const Tensor& x, const Tensor& g) {
+  if (!dy.is_cuda() || x.device() != dy.device() || dy.scalar_type() != x.scalar_type() ||
+      (code(dy) != MI_BF16 && code(dy) != MI_F16) ||
+      !lib.mi_wgrad_suits(dy.size(0), dy.size(1), x.size(1)))
+    return Tensor();
+  for (const Tensor* t : {&dy, &x})
+    if (t->stride(1) != 1 || t->stride(0) < t->size(1) || t->stride(0) >= 1 << 24 ||
+        t->stride(0) % 8 || t->size(1) % 8 || (uintptr_t)t->data_ptr() % 16)
+      return Tensor();
+  if (g.defined() && (g.scalar_type() != dy.scalar_type() || g.device() != dy.device() ||
+                      (uintptr_t)g.data_ptr() % 8))
+    return Tensor();
+  const int64_t n = lib.mi_wgrad_workspace(dy.size(0), dy.size(1), x.size(1));
+  Tensor dw = g.defined() ? g : empty({dy.size(1), x.size(1)}, dy), ws = empty_f32({n}, dy);
+  check(lib.mi_wgrad(dt(dy), dy.size(0), dy.size(1), x.size(1), dy.data_ptr(), dy.stride(0),
+                     x.data_ptr(), x.stride(0), dw.data_ptr(), g.defined(), ws.data_ptr<float>(),
+                     n, stream(dy)),
+        "mi_wgrad");
+  return dw;
+}
+
 struct LinearGradInto : torch::autograd::Function<LinearGradInto> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, bool into) {
     ctx->save_for_backward({x, w});
+    ctx->saved_data["into"] = into;
     return at::linear(x, w);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
     const Tensor &x = s[0], &w = s[1], &gy = grads[0];
     const Tensor gx = ctx->needs_input_grad(0) ? gy.matmul(w) : Tensor();
-    if (!ctx->needs_input_grad(1)) return {gx, Tensor()};
+    if (!ctx->needs_input_grad(1)) return {gx, Tensor(), Tensor()};
     const Tensor gy2 = gy.reshape({-1, gy.size(-1)}), x2 = x.reshape({-1, x.size(-1)});
-    Tensor g = w.grad();
-    if (!g.defined() || at::GradMode::is_enabled() || g.scalar_type() != gy.scalar_type() ||
-        g.sizes() != w.sizes() || !g.is_contiguous())
-      return {gx, gy2.t().matmul(x2)};
-    g.addmm_(gy2.t(), x2);
-    return {gx, Tensor()};
+    if (at::GradMode::is_enabled()) return {gx, gy2.t().matmul(x2), Tensor()};
+    Tensor g = ctx->saved_data["into"].toBool() ? w.grad() : Tensor();
+    if (!g.defined() || g.scalar_type() != gy.scalar_type() || g.sizes() != w.sizes() ||
+        !g.is_contiguous()) {
+      const Tensor dw = wgrad(gy2, x2, Tensor());
+      return {gx, dw.defined() ? dw : gy2.t().matmul(x2), Tensor()};
+    }
+    if (!wgrad(gy2, x2, g).defined()) g.addmm_(gy2.t(), x2);
+    return {gx, Tensor(), Tensor()};
   }
 };
 
@@ -723,9 +750,10 @@ PyObject* py_swiglu(PyObject*, Args a, Py_ssize_t n) {
 PyObject* py_linear_into_grad(PyObject*, Args a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Tensor x, w;
-  PLAIN(n == 2 && plain(a[0], x) && plain(a[1], w) && plain_context() && x.dim() >= 1 &&
-        w.dim() == 2 && x.size(-1) == w.size(1) && one_device(x, w));
-  return THPVariable_Wrap(released([&] { return LinearGradInto::apply(x, w); }));
+  bool into;
+  PLAIN(n == 3 && plain(a[0], x) && plain(a[1], w) && plain_context() && x.dim() >= 1 &&
+        w.dim() == 2 && x.size(-1) == w.size(1) && one_device(x, w) && truth(a[2], into));
+  return THPVariable_Wrap(released([&] { return LinearGradInto::apply(x, w, into); }));
   END_HANDLE_TH_ERRORS
 }
 

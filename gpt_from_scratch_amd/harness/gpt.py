@@ -57,12 +57,14 @@ from ..rope import apply_rope_qk
 
 
 class _LinearGradInto(torch.autograd.Function):
-    """``F.linear(x, w)`` whose weight gradient the GEMM accumulates itself into
-    ``w.grad`` when that already exists (the optimizer's flat gradient buffer):
-    ``w.grad.addmm_(gy^T, x)``, beta = 1 in the GEMM's epilogue, instead of a
-    separate gradient tensor that autograd then adds into the buffer with one
-    more pass over it.  Without a usable ``w.grad`` (none yet, another dtype or
-    layout, or a double backward) the gradient is returned as F.linear's is.
+    """``F.linear(x, w)`` whose weight gradient the product accumulates itself
+    into ``w.grad`` when that already exists (the optimizer's flat gradient
+    buffer), instead of a separate gradient tensor that autograd then adds into
+    the buffer with one more pass over it.  Long products of few output tiles
+    run in the library's own kernel (mi_wgrad, tokens split over the chip),
+    others as ``w.grad.addmm_(gy^T, x)``, beta = 1 in the GEMM's epilogue.
+    Without a usable ``w.grad`` (none yet, another dtype or layout, or a double
+    backward), or with ``into=False``, the gradient is returned as F.linear's is.
 
     The fused form rounds once, round(g + acc), where autograd's add rounds the
     gradient first, round(round(g) + acc).  The two agree bit for bit only when
@@ -72,8 +74,9 @@ class _LinearGradInto(torch.autograd.Function):
     a weight used twice in one graph the results would differ in the last bit."""
 
     @staticmethod
-    def forward(ctx, x, w):
+    def forward(ctx, x, w, into=True):
         ctx.save_for_backward(x, w)
+        ctx.into = into
         return F.linear(x, w)
 
     @staticmethod
@@ -81,20 +84,27 @@ class _LinearGradInto(torch.autograd.Function):
         x, w = ctx.saved_tensors
         gx = gy.matmul(w) if ctx.needs_input_grad[0] else None
         if not ctx.needs_input_grad[1]:
-            return gx, None
+            return gx, None, None
         gy2 = gy.reshape(-1, gy.shape[-1])
         x2 = x.reshape(-1, x.shape[-1])
-        g = w.grad
-        if (g is None or torch.is_grad_enabled() or g.dtype != gy.dtype or g.shape != w.shape
-                or not g.is_contiguous()):
-            return gx, gy2.t().matmul(x2)
-        g.addmm_(gy2.t(), x2)
-        return gx, None
+        if torch.is_grad_enabled():
+            return gx, gy2.t().matmul(x2), None
+        g = w.grad if ctx.into else None
+        if g is None or g.dtype != gy.dtype or g.shape != w.shape or not g.is_contiguous():
+            dw = _lib.wgrad(gy2, x2)
+            return gx, gy2.t().matmul(x2) if dw is None else dw, None
+        if _lib.wgrad(gy2, x2, g) is None:
+            g.addmm_(gy2.t(), x2)
+        return gx, None, None
+
+
+def _linear(x, w, into=False):
+    y = _lib.ops().linear_into_grad(x, w, into) if x.is_cuda else None
+    return _LinearGradInto.apply(x, w, into) if y is None else y
 
 
 def _linear_into_grad(x, w):
-    y = _lib.ops().linear_into_grad(x, w) if x.is_cuda else None
-    return _LinearGradInto.apply(x, w) if y is None else y
+    return _linear(x, w, True)
 
 
 @dataclasses.dataclass
@@ -221,7 +231,7 @@ class GPT(nn.Module):
         # norms' by their backward kernels, into the optimizer's gradient buffer
         # (not with eager_ops, which keeps the reference's ops throughout)
         into = gemm_grad_accumulate and not eager_ops
-        self.lin = _linear_into_grad if into else F.linear
+        self.lin = F.linear if eager_ops else _linear_into_grad if into else _linear
         emb = torch.empty(cfg.vocab_size, cfg.hidden_size, device=device, dtype=torch.float32)
         nn.init.xavier_uniform_(emb)
         self.embedding = nn.Parameter(emb)

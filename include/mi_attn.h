@@ -384,6 +384,23 @@ mi_status mi_swiglu_bwd(mi_dtype dtype, int64_t rows, int64_t inter, const void*
                         int64_t gate_up_row_stride, const void* dout, int64_t dout_row_stride,
                         void* dgate_up, int64_t dgate_up_row_stride, void* stream);
 
+/* Weight gradient of a projection y = x W^T: dweight[out, in] =
+ * round(dy[rows, out]^T x[rows, in]), or with `accumulate` the same added to
+ * dweight before the rounding; summed in fp32 and rounded once (the backward of
+ * core/tensor_parallel/layers.py's projections at one rank).
+ * bf16 or f16; dy and x rows `*_row_stride` elements apart, every row 16-byte
+ * aligned and of a multiple of 8 elements; dweight dense.  workspace:
+ * mi_wgrad_workspace(rows, out, in) floats, 16-byte aligned, contents
+ * irrelevant.  mi_wgrad_suits: whether these sizes are ones it is built for
+ * (long rows, few tiles of dweight); others are correct, but a general GEMM is
+ * faster. */
+int mi_wgrad_suits(int64_t rows, int64_t out_features, int64_t in_features);
+int64_t mi_wgrad_workspace(int64_t rows, int64_t out_features, int64_t in_features);
+mi_status mi_wgrad(mi_dtype dtype, int64_t rows, int64_t out_features, int64_t in_features,
+                   const void* dy, int64_t dy_row_stride, const void* x, int64_t x_row_stride,
+                   void* dweight, int accumulate, float* workspace, int64_t workspace_elems,
+                   void* stream);
+
 /* fp32 elements of workspace mi_grad_sumsq needs (result in element 0). */
 int64_t mi_adamw_workspace(void);
 
