@@ -6,6 +6,7 @@
 // message.  No allocation and no synchronisation.  Global mutable state: the
 // thread-local error text, and the forward's per-device cache of the compute
 // unit count (atomic entries, written once per device with the same value).
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <initializer_list>
@@ -794,7 +795,7 @@ mi_status mi_rmsnorm_add_fwd(mi_dtype x_dtype, mi_dtype w_dtype, int64_t rows, i
 
 int64_t mi_rmsnorm_bwd_workspace(int64_t rows, int64_t hidden) {
   if (rows <= 0 || hidden <= 0) return 0;
-  return mi::rmsnorm_parts(rows) * hidden;
+  return mi::rmsnorm_parts(rows, hidden) * hidden;
 }
 
 static mi_status rms_bwd(mi_dtype x_dtype, mi_dtype w_dtype, int64_t rows, int64_t hidden,
@@ -820,7 +821,7 @@ static mi_status rms_bwd(mi_dtype x_dtype, mi_dtype w_dtype, int64_t rows, int64
       ((uintptr_t)dy) % elem_size(y_dtype) || ((uintptr_t)dx) % elem_size(x_dtype) ||
       ((uintptr_t)dweight) % elem_size(w_dtype))
     return fail(MI_ERR_INVALID_ARGUMENT, "rstd / dy / dx / dweight / workspace: misaligned");
-  const int64_t need = mi_rmsnorm_bwd_workspace(rows, hidden);
+  const int64_t need = mi::rmsnorm_min_parts(rows) * hidden;
   if (workspace_elems < need)
     return fail(MI_ERR_INVALID_ARGUMENT, "workspace holds %lld floats, %lld needed",
                 (long long)workspace_elems, (long long)need);
@@ -832,7 +833,7 @@ static mi_status rms_bwd(mi_dtype x_dtype, mi_dtype w_dtype, int64_t rows, int64
   a.dw = dweight;
   a.dw_acc = dw_acc ? 1 : 0;
   a.partial = workspace;
-  a.parts = (int)mi::rmsnorm_parts(rows);
+  a.parts = (int)std::min(mi::rmsnorm_parts(rows, hidden), workspace_elems / hidden);
   bool vec = rms_vec_ok(hidden, {{x, x_row_stride}, {dy, dy_row_stride}, {dx, dx_row_stride}},
                         {{x, elem_size(x_dtype)}, {dy, elem_size(y_dtype)},
                          {dx, elem_size(x_dtype)}, {weight, elem_size(w_dtype)}});

@@ -130,8 +130,10 @@ struct RmsArgs {
   int64_t dsum_stride;
 };
 
-// Number of dw partial rows the backward uses for `rows` rows (<= 256).
-int64_t rmsnorm_parts(int64_t rows);
+// Number of dw partial rows the backward uses (<= 256) where the workspace holds
+// them, and the fewest that it runs with.
+int64_t rmsnorm_parts(int64_t rows, int64_t hidden);
+int64_t rmsnorm_min_parts(int64_t rows);
 hipError_t launch_rmsnorm_fwd(int x_dtype, int w_dtype, const RmsArgs& a, bool vec,
                               hipStream_t st);
 hipError_t launch_rmsnorm_bwd(int x_dtype, int w_dtype, const RmsArgs& a, bool vec,

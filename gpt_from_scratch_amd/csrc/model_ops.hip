@@ -18,6 +18,9 @@
 // 16-byte vectors and a scalar tail.
 //
 // RMSNorm (core/normalization.py:13-25): further below.
+#include <algorithm>
+#include <utility>
+
 #include "mi_device.h"
 #include "mi_kernels.h"
 
@@ -921,6 +924,266 @@ __global__ __launch_bounds__(256) void rmsnorm_dw_partial_scalar_kernel(RmsArgs 
   a.partial[(int64_t)blockIdx.y * a.hidden + col] = t;
 }
 
+// Wide rows: one workgroup of RMS_WT threads per row, each thread C chunks of 8
+// elements.  A wave per row needs H / 64 values per lane in registers for one
+// row (the backward, at H > 2048, more than there are); here it is 8 or 16, so
+// many rows are in flight, and a dw column belongs to one thread: no reduction
+// over waves.  Bound: HBM.  us, forward / backward with the residual add, from
+// HBM, before (a wave per row; backward: scalar kernels) -> here:
+//   bf16 [8192, 2048]   25.7 / -     -> 24.4 / -
+//   bf16 [4096, 4096]   35.3 / 86.8  -> 23.9 / 29.4 (5.6 / 4.6 TB/s)
+//   bf16 [2048, 8192]  102.8 / 125.3 -> 24.8 / 30.6
+//   bf16 [4096, 4095]   62.9 / 86.6  -> 28.8 / 32.1
+//   fp32 [2048, 8192]  114.3 / 149.8 -> 54.3 / 57.0
+// Elements of chunk c of thread t: 8 (c RMS_WT + t) + 0..7, in one 16-byte
+// access at V = 8 and two of 4 elements at V = 4 (the same sums); at V = 1, rows
+// that are aligned to less, (8 c + e) RMS_WT + t.  A thread reads and writes the
+// same elements, so outputs may alias inputs.
+constexpr int RMS_WT = 512;
+constexpr int64_t RMS_WIDE_MAX = 2 * 8 * RMS_WT;
+
+// For fp16, v rounded to fp32 before whatever rounds it to fp16: the compiler
+// may otherwise fuse the two into one rounding, in one kernel and not another.
+template <int DT>
+__device__ __forceinline__ float pinned(float v) {
+  if constexpr (DT == 1) asm("" : "+v"(v));
+  return v;
+}
+
+// One chunk of a row as loaded; get() puts zeros past the row's end.  Rows of 4:
+// the two halves under one branch in the forward ([8192, 2044] bf16 with the add:
+// 31.3 us, in two 35.7), under one each in the backward ([4096, 2052]: 24.4, 36.6).
+template <int DT, int V, bool FWD, bool NT = true>
+struct WideChunk {
+  typedef typename Store<DT>::type T;
+  typedef typename Packed4<DT>::type P;
+  P q[2];
+  T raw[8];
+  __device__ __forceinline__ void load(const void* row, int c, int h) {
+    const int t = threadIdx.x;
+    if constexpr (V == 1) {
+      // unconditional, at a clamped index: a branch per element would wait for each
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int i = (8 * c + e) * RMS_WT + t;
+        raw[e] = ((const T*)row)[(unsigned)(i < h ? i : h - 1)];
+      }
+    } else {
+      const int i = 8 * (c * RMS_WT + t);
+      if constexpr (V == 8 && DT != 0) {
+        const u32x4* p = (const u32x4*)((const T*)row + i);
+        u32x4 w = {0, 0, 0, 0};
+        if (i < h) w = NT ? __builtin_nontemporal_load(p) : *p;
+        q[0] = P{w[0], w[1]};
+        q[1] = P{w[2], w[3]};
+      } else if constexpr (V == 8 || FWD) {
+        q[0] = q[1] = P{};
+        if ((V == 8 ? i : i + 4) < h) {
+          q[0] = ld4_packed<DT, NT>(row, i);
+          q[1] = ld4_packed<DT, NT>(row, i + 4);
+        } else if (V == 4 && i < h) {
+          q[0] = ld4_packed<DT, NT>(row, i);
+        }
+      } else {
+        q[0] = q[1] = P{};
+        if (i < h) q[0] = ld4_packed<DT, NT>(row, i);
+        if (i + 4 < h) q[1] = ld4_packed<DT, NT>(row, i + 4);
+      }
+    }
+  }
+  __device__ __forceinline__ void get(float (&v)[8], int c, int h) const {
+    if constexpr (V == 1) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int i = (8 * c + e) * RMS_WT + (int)threadIdx.x;
+        v[e] = i < h ? Store<DT>::ld(raw, e) : 0.f;
+      }
+    } else {
+      float u[2][4];
+      unpack4<DT>(q[0], u[0]);
+      unpack4<DT>(q[1], u[1]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = u[e >> 2][e & 3];
+    }
+  }
+};
+
+template <int DT, int V>
+__device__ __forceinline__ void wide_store(void* row, int c, int h, const float (&v)[8]) {
+  const int t = threadIdx.x;
+  if constexpr (V == 1) {
+    typedef typename Store<DT>::type T;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int i = (8 * c + e) * RMS_WT + t;
+      if (i < h) Store<DT>::st((T*)row, i, v[e]);
+    }
+  } else {
+    const int i = 8 * (c * RMS_WT + t);
+    if constexpr (V == 8 && DT != 0) {
+      if (i < h) st8<DT, true>(row, i, v);
+    } else {
+      // both halves of a line's sector next to each other: in two branches the
+      // fp32 forward at [2048, 8192] took 78.6 us, not 54.3
+      const float u[2][4] = {{v[0], v[1], v[2], v[3]}, {v[4], v[5], v[6], v[7]}};
+      const int last = V == 8 ? i : i + 4;
+      if (last < h) {
+        st4<DT, true>(row, i, u[0]);
+        st4<DT, true>(row, i + 4, u[1]);
+      } else if (V == 4 && i < h) {
+        st4<DT, true>(row, i, u[0]);
+      }
+    }
+  }
+}
+
+// Sum over the workgroup, the same bits in every thread; `slot` alternates
+// between calls.  Only LDS is fenced: loads of the next row stay in flight.
+__device__ __forceinline__ float wide_sum(float v, float (&red)[2][RMS_WT / 64], int slot) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[slot][threadIdx.x >> 6] = v;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  float t = 0.f;
+#pragma unroll
+  for (int k = 0; k < RMS_WT / 64; ++k) t += red[slot][k];
+  return t;
+}
+
+template <int DT, int WDT, int C, bool ADD, int V>
+__global__ __launch_bounds__(RMS_WT) void rmsnorm_fwd_wide_kernel(RmsArgs a) {
+  constexpr int YDT = RmsTypes<DT, WDT>::YDT;
+  __shared__ float red[2][RMS_WT / 64];
+  const int h = (int)a.hidden;
+  int slot = 0;
+  for (int64_t row = blockIdx.x; row < a.rows; row += gridDim.x, slot ^= 1) {
+    WideChunk<DT, V, true> xq[C], rq[ADD ? C : 1];
+    WideChunk<WDT, V, true, false> wq[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      xq[c].load(row_ptr<DT>(a.x, row, a.x_stride), c, h);
+      if constexpr (ADD) rq[c].load(row_ptr<DT>(a.res, row, a.res_stride), c, h);
+      wq[c].load(a.w, c, h);
+    }
+    float v[C][8], ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      xq[c].get(v[c], c, h);
+      if constexpr (ADD) {
+        float r[8];
+        rq[c].get(r, c, h);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[c][e] = round_to<DT>(pinned<DT>(v[c][e] + r[e]));
+        wide_store<DT, V>(row_ptr<DT>(a.sum, row, a.sum_stride), c, h, v[c]);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(v[c][e], v[c][e], ss);
+    }
+    ss = wide_sum(ss, red, slot);
+    const float r = __builtin_amdgcn_rsqf(ss / (float)h + a.eps);
+    if (threadIdx.x == 0) a.rstd[row] = r;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      float w[8], y[8];
+      wq[c].get(w, c, h);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = round_to<DT>(pinned<DT>(v[c][e] * r)) * w[e];
+      wide_store<YDT, V>(row_ptr<YDT>(a.y, row, a.y_stride), c, h, y);
+    }
+  }
+}
+
+// dx of rows blockIdx.x, + gridDim.x, ..., the next row's loads in flight while
+// a row is finished, and this workgroup's partial dw into partial[blockIdx.x].
+template <int DT, int WDT, int C, bool ADD, int V>
+__global__ __launch_bounds__(RMS_WT) void rmsnorm_bwd_wide_kernel(RmsArgs a) {
+  constexpr int YDT = RmsTypes<DT, WDT>::YDT;
+  __shared__ float red[2][RMS_WT / 64];
+  const int h = (int)a.hidden;
+  const float inv_h = 1.f / (float)h;
+  float acc[C][8], w[C][8];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    WideChunk<WDT, V, false, false> q;
+    q.load(a.w, c, h);
+    q.get(w[c], c, h);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[c][e] = 0.f;
+  }
+  struct Row {
+    WideChunk<DT, V, false> x[C], ds[ADD ? C : 1];
+    WideChunk<YDT, V, false> dy[C];
+    float r;
+  };
+  auto load = [&](Row& q, int64_t row) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      q.x[c].load(row_ptr<DT>(a.x, row, a.x_stride), c, h);
+      q.dy[c].load(row_ptr<YDT>(a.dy, row, a.dy_stride), c, h);
+      if constexpr (ADD) q.ds[c].load(row_ptr<DT>(a.dsum, row, a.dsum_stride), c, h);
+    }
+    q.r = a.rstd[row];
+  };
+  auto finish = [&](const Row& q, int64_t row, int slot) __attribute__((always_inline)) {
+    float x[C][8], dn[C][8], s = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      q.x[c].get(x[c], c, h);
+      q.dy[c].get(dn[c], c, h);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        acc[c][e] = __builtin_fmaf(dn[c][e], round_to<DT>(pinned<DT>(x[c][e] * q.r)), acc[c][e]);
+        dn[c][e] *= w[c][e];
+        s = __builtin_fmaf(dn[c][e], x[c][e], s);
+      }
+    }
+    const float k = q.r * q.r * q.r * wide_sum(s, red, slot) * inv_h;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      float d[8], ds[8];
+      if constexpr (ADD) q.ds[c].get(ds, c, h);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        d[e] = pinned<DT>(__builtin_fmaf(q.r, dn[c][e], -x[c][e] * k));
+        if constexpr (ADD) d[e] = pinned<DT>(round_to<DT>(d[e]) + ds[e]);
+      }
+      wide_store<DT, V>(row_ptr<DT>(a.dx, row, a.dx_stride), c, h, d);
+    }
+  };
+  const int64_t step = gridDim.x;
+  int64_t row = blockIdx.x;
+  if constexpr (C == 2 && V == 1) {
+    // two rows of 2 x 8 unpacked elements per thread would not fit the registers
+    Row q;
+    for (int slot = 0; row < a.rows; row += step, slot ^= 1) {
+      load(q, row);
+      finish(q, row, slot);
+    }
+  } else {
+    Row q0, q1;
+    if (row < a.rows) load(q0, row);
+    for (; row < a.rows; row += 2 * step) {
+      const bool more = row + step < a.rows;
+      if (more) load(q1, row + step);
+      finish(q0, row, 0);
+      if (!more) break;
+      if (row + 2 * step < a.rows) load(q0, row + 2 * step);
+      finish(q1, row + step, 1);
+    }
+  }
+  float* part = a.partial + (int64_t)blockIdx.x * h;
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; e += V == 1 ? 1 : 4) {
+      const int t = threadIdx.x;
+      const int i = V == 1 ? (8 * c + e) * RMS_WT + t : 8 * (c * RMS_WT + t) + e;
+      // the workspace may be aligned to 4 bytes only
+      if (i < h) __builtin_memcpy(part + i, &acc[c][e], V == 1 ? 4 : 16);
+    }
+}
+
 // Columns per workgroup of the dw reduction (16 partial groups each): 16
 // puts H / 16 workgroups on the [parts, H] partials (48 at H = 768), ~0.5 us
 // faster per backward at config 5 than 64 columns (12 workgroups); 8 and 32
@@ -957,6 +1220,23 @@ __global__ __launch_bounds__(16 * DW_COLS) void rmsnorm_dw_reduce_kernel(RmsArgs
 // holds dy and the dw partial in registers, H <= 64 * 4 * 8 (beyond, it spills).
 constexpr int64_t RMS_VEC_FWD_MAX = 4096, RMS_VEC_BWD_MAX = 2048;
 
+// Whether a row is a workgroup's (the wide kernels) and not a wave's: up to what
+// 16 elements per thread cover, and from where the wave's registers run short.
+// The backward's from RMS_VEC_BWD_MAX, where only the scalar kernels are left (at
+// [8192, 2048] bf16 the two tie: 37.1 against 35.1 us with the add, 31.1 against
+// 32.2 without).  The forward's, us with the add / without, wave against workgroup:
+// 16-bit [8192, 1536] 19.4 / 10.1 against 19.9 / 15.5, [8192, 1600] 21.6 / 16.6
+// against 20.4 / 15.9, so from 1536 (rows of 4, [8192, 2044]: 34.1 / 23.3 against
+// 31.3 / 18.2, with an fp32 weight 36.1 / 25.2 against 37.3 / 25.1: the same line,
+// so that a row's bits do not depend on its alignment to 4 or 8); fp32 [4096, 4096] 48.5 / 27.8 against 52.3 /
+// 28.6, so as long as the vector kernels go; scalar rows [8192, 1537] 31.1 / 20.2
+// against 35.1 / 20.1, [8192, 2047] 41.7 / 25.2 against 37.0 / 20.6.
+bool rms_wide(bool fwd, int dt, const RmsArgs& a, bool vec) {
+  if (a.hidden > RMS_WIDE_MAX) return false;
+  if (!fwd || !vec) return a.hidden > RMS_VEC_BWD_MAX;
+  return a.hidden > (dt == 0 ? RMS_VEC_FWD_MAX : 1536);
+}
+
 template <int DT, int WDT, int C, bool ADD>
 void launch_rms_vec(bool fwd, const RmsArgs& a, hipStream_t st) {
   if (fwd)
@@ -967,9 +1247,57 @@ void launch_rms_vec(bool fwd, const RmsArgs& a, hipStream_t st) {
                        dim3(64 * RmsBwdCfg<C>::W), 0, st, a);
 }
 
+// Rows that one 16-byte access per 8 elements can read and write.
+bool rows_of_8(const RmsArgs& a) {
+  if (a.hidden % 8) return false;
+  const std::pair<const void*, int64_t> rows[] = {
+      {a.x, a.x_stride},     {a.y, a.y_stride},     {a.dy, a.dy_stride},     {a.dx, a.dx_stride},
+      {a.res, a.res_stride}, {a.sum, a.sum_stride}, {a.dsum, a.dsum_stride}, {a.w, 0}};
+  for (const auto& r : rows)
+    if (r.first && (((uintptr_t)r.first) % 16 || r.second % 8)) return false;
+  return true;
+}
+
+template <int DT, int WDT, bool ADD, int C, int V>
+void launch_rms_wide_cv(bool fwd, const RmsArgs& a, hipStream_t st) {
+  // a grid's threads must stay below 2^32: more rows are looped over
+  const unsigned rows = (unsigned)std::min<int64_t>(a.rows, 1 << 22);
+  if (fwd)
+    hipLaunchKernelGGL((rmsnorm_fwd_wide_kernel<DT, WDT, C, ADD, V>), dim3(rows), dim3(RMS_WT), 0,
+                       st, a);
+  else
+    hipLaunchKernelGGL((rmsnorm_bwd_wide_kernel<DT, WDT, C, ADD, V>), dim3((unsigned)a.parts),
+                       dim3(RMS_WT), 0, st, a);
+}
+
+template <int DT, int WDT, bool ADD, int C>
+void launch_rms_wide_c(bool fwd, const RmsArgs& a, bool vec, hipStream_t st) {
+  if (!vec) return launch_rms_wide_cv<DT, WDT, ADD, C, 1>(fwd, a, st);
+  if (rows_of_8(a)) return launch_rms_wide_cv<DT, WDT, ADD, C, 8>(fwd, a, st);
+  launch_rms_wide_cv<DT, WDT, ADD, C, 4>(fwd, a, st);
+}
+
+template <int DT, int WDT, bool ADD>
+void launch_rms_wide(bool fwd, const RmsArgs& a, bool vec, hipStream_t st) {
+  if (a.hidden <= 8 * RMS_WT) launch_rms_wide_c<DT, WDT, ADD, 1>(fwd, a, vec, st);
+  else launch_rms_wide_c<DT, WDT, ADD, 2>(fwd, a, vec, st);
+}
+
+template <int WDT>
+void launch_dw_reduce(const RmsArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((rmsnorm_dw_reduce_kernel<WDT>),
+                     dim3((unsigned)((a.hidden + DW_COLS - 1) / DW_COLS)), dim3(16 * DW_COLS), 0,
+                     st, a);
+}
+
 template <int DT, int WDT, bool ADD>
 hipError_t launch_rms_dt(bool fwd, const RmsArgs& a, bool vec, hipStream_t st) {
   const int64_t nq = a.hidden / 4;
+  if (rms_wide(fwd, DT, a, vec)) {
+    launch_rms_wide<DT, WDT, ADD>(fwd, a, vec, st);
+    if (!fwd) launch_dw_reduce<WDT>(a, st);
+    return hipGetLastError();
+  }
   if (a.hidden > (fwd ? RMS_VEC_FWD_MAX : RMS_VEC_BWD_MAX)) vec = false;
   // bf16 only: for fp16 the backend fuses some of a row's x * r products with
   // their conversion into one v_fma_mixlo_f16 (a single rounding of the exact
@@ -983,10 +1311,7 @@ hipError_t launch_rms_dt(bool fwd, const RmsArgs& a, bool vec, hipStream_t st) {
       else if (n8 <= 64) hipLaunchKernelGGL((rmsnorm_fwd_v16_kernel<DT, WDT, 2, ADD>), grid, dim3(256), 0, st, a);
       else if (n8 <= 96) hipLaunchKernelGGL((rmsnorm_fwd_v16_kernel<DT, WDT, 3, ADD>), grid, dim3(256), 0, st, a);
       else if (n8 <= 128) hipLaunchKernelGGL((rmsnorm_fwd_v16_kernel<DT, WDT, 4, ADD>), grid, dim3(256), 0, st, a);
-      else if (n8 <= 192) hipLaunchKernelGGL((rmsnorm_fwd_v16_kernel<DT, WDT, 6, ADD>), grid, dim3(256), 0, st, a);
-      else if (n8 <= 256) hipLaunchKernelGGL((rmsnorm_fwd_v16_kernel<DT, WDT, 8, ADD>), grid, dim3(256), 0, st, a);
-      else if (n8 <= 384) hipLaunchKernelGGL((rmsnorm_fwd_v16_kernel<DT, WDT, 12, ADD>), grid, dim3(256), 0, st, a);
-      else hipLaunchKernelGGL((rmsnorm_fwd_v16_kernel<DT, WDT, 16, ADD>), grid, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL((rmsnorm_fwd_v16_kernel<DT, WDT, 6, ADD>), grid, dim3(256), 0, st, a);
       return hipGetLastError();
     }
   }
@@ -998,8 +1323,10 @@ hipError_t launch_rms_dt(bool fwd, const RmsArgs& a, bool vec, hipStream_t st) {
     else if (nq <= 256) launch_rms_vec<DT, WDT, 4, ADD>(fwd, a, st);
     else if (nq <= 384) launch_rms_vec<DT, WDT, 6, ADD>(fwd, a, st);
     else if (nq <= 512) launch_rms_vec<DT, WDT, 8, ADD>(fwd, a, st);
-    else if (nq <= 768) launch_rms_vec<DT, WDT, 12, ADD>(fwd, a, st);
-    else launch_rms_vec<DT, WDT, 16, ADD>(fwd, a, st);
+    else if constexpr (DT == 0) {
+      if (nq <= 768) launch_rms_vec<DT, WDT, 12, ADD>(fwd, a, st);
+      else launch_rms_vec<DT, WDT, 16, ADD>(fwd, a, st);
+    }
   } else if (fwd) {
     hipLaunchKernelGGL((rmsnorm_fwd_scalar_kernel<DT, WDT, ADD>),
                        dim3((unsigned)((a.rows + 3) / 4)), dim3(256), 0, st, a);
@@ -1012,10 +1339,7 @@ hipError_t launch_rms_dt(bool fwd, const RmsArgs& a, bool vec, hipStream_t st) {
     hipLaunchKernelGGL((rmsnorm_bwd_dx_scalar_kernel<DT, WDT, ADD>),
                        dim3((unsigned)((a.rows + 3) / 4)), dim3(256), 0, st, a);
   }
-  if (!fwd)
-    hipLaunchKernelGGL((rmsnorm_dw_reduce_kernel<WDT>),
-                       dim3((unsigned)((a.hidden + DW_COLS - 1) / DW_COLS)),
-                       dim3(16 * DW_COLS), 0, st, a);
+  if (!fwd) launch_dw_reduce<WDT>(a, st);
   return hipGetLastError();
 }
 
@@ -1038,9 +1362,14 @@ hipError_t launch_rms(bool fwd, int x_dtype, int w_dtype, const RmsArgs& a, bool
 
 }  // namespace
 
-int64_t rmsnorm_parts(int64_t rows) {
-  const int64_t p = (rows + RMS_PARTS_ROWS - 1) / RMS_PARTS_ROWS;
-  return p < 1 ? 1 : (p > 256 ? 256 : p);
+// The wide backward's workgroups take one row at a time, the others' several.
+int64_t rmsnorm_parts(int64_t rows, int64_t hidden) {
+  const int64_t per = hidden > RMS_VEC_BWD_MAX && hidden <= RMS_WIDE_MAX ? 2 : RMS_PARTS_ROWS;
+  return std::clamp<int64_t>((rows + per - 1) / per, 1, 256);
+}
+
+int64_t rmsnorm_min_parts(int64_t rows) {
+  return std::clamp<int64_t>((rows + RMS_PARTS_ROWS - 1) / RMS_PARTS_ROWS, 1, 256);
 }
 
 hipError_t launch_rmsnorm_fwd(int x_dtype, int w_dtype, const RmsArgs& a, bool vec,
