@@ -441,6 +441,13 @@ def wgrad(dy, x, dweight=None):
     if dy.device.type != "cuda" or x.device != dy.device or dy.dtype != x.dtype \
             or dy.dtype not in (torch.bfloat16, torch.float16):
         return None
+    # the C ABI takes the sizes from dy and x: operands that do not fit each other
+    # are left to the general GEMM, which refuses them
+    if dy.dim() != 2 or x.dim() != 2 or x.shape[0] != dy.shape[0]:
+        return None
+    if dweight is not None and (tuple(dweight.shape) != (dy.shape[1], x.shape[1])
+                                or not dweight.is_contiguous()):
+        return None
     rows, out = dy.shape
     if not lib().mi_wgrad_suits(rows, out, x.shape[1]):
         return None

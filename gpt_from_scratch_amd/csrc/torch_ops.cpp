@@ -557,8 +557,14 @@ struct SwiGLU : torch::autograd::Function<SwiGLU> {
 };
 
 // dy^T x added to g, or in a new tensor (_lib.wgrad); undefined where a general
-// GEMM is to be used.
+// GEMM is to be used.  The C ABI takes the sizes from dy and x: operands that do
+// not fit each other (a saved x may have changed) are left to the GEMM, which
+// refuses them.
 Tensor wgrad(const Tensor& dy, const Tensor& x, const Tensor& g) {
+  if (dy.dim() != 2 || x.dim() != 2 || x.size(0) != dy.size(0) ||
+      (g.defined() &&
+       (g.dim() != 2 || g.size(0) != dy.size(1) || g.size(1) != x.size(1) || !g.is_contiguous())))
+    return Tensor();
   if (!dy.is_cuda() || x.device() != dy.device() || dy.scalar_type() != x.scalar_type() ||
       (code(dy) != MI_BF16 && code(dy) != MI_F16) ||
       !lib.mi_wgrad_suits(dy.size(0), dy.size(1), x.size(1)))

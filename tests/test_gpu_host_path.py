@@ -177,8 +177,6 @@ def test_saved_tensor_hooks_and_in_place_checks(gpu):
 def test_hooks_that_change_a_saved_tensor_are_refused(gpu):
     """Shapes and devices of what comes back are checked before any launch."""
     for name, (fn, cls, tensors, args) in _cases().items():
-        if name.startswith("linear"):
-            continue  # torch's own products check theirs
         for bad in (lambda t: t[:1] if t.dim() else t, lambda t: t.cpu()):
             xs = [_leaf(t, True) for t in tensors]
             with torch.autograd.graph.saved_tensors_hooks(lambda t: t, bad):

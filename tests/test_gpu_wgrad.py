@@ -95,6 +95,28 @@ def test_what_the_projection_hands_over(gpu):
     assert suits == [True, True, False, False]
 
 
+def test_operands_that_no_longer_fit_are_refused(gpu):
+    """A saved x that a hook changed, or a gradient of other sizes: torch's
+    products refuse them, as at sizes that mi_wgrad does not take, and the
+    gradient is left alone."""
+    from gpt_from_scratch_amd.harness import gpt
+    M, N, K = 600, 136, 64
+    x, w, gy = seeded((M, K), 1).to(gpu), seeded((N, K), 2).to(gpu), seeded((M, N), 3).to(gpu)
+    changed = [lambda t: t[:300], lambda t: t.repeat(2, 1), lambda t: t.repeat(1, 2),
+               lambda t: t[:, :32].contiguous()]
+    for fn in (gpt._linear, gpt._LinearGradInto.apply):
+        for into in (True, False):
+            for bad in changed:
+                xl, wl = x.clone(), w.clone().requires_grad_()  # x needs no gradient: only dw runs
+                wl.grad = torch.ones_like(wl)
+                with torch.autograd.graph.saved_tensors_hooks(
+                        lambda t: t, lambda t: bad(t) if t.shape == (M, K) else t):
+                    y = fn(xl, wl, into)
+                    with pytest.raises(RuntimeError):
+                        y.backward(gy)
+                assert bool((wl.grad == 1).all())
+
+
 def test_refusals(gpu):
     from gpt_from_scratch_amd import _lib
     dy, x = seeded((512, 136), 1).to(gpu), seeded((512, 64), 2).to(gpu)

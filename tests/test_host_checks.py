@@ -1,0 +1,61 @@
+"""What the Python side refuses or hands on before any launch (no GPU needed)."""
+import pytest
+import torch
+
+from gpt_from_scratch_amd import _lib
+
+
+class _OnGpu:
+    """The attributes of a GPU tensor that _lib.wgrad looks at."""
+
+    device = torch.device("cuda:0")
+
+    def __init__(self, *shape, dtype=torch.bfloat16, stride=None):
+        self.shape, self.dtype = shape, dtype
+        self._stride = stride or tuple(
+            torch.empty(shape, dtype=dtype, device="meta").stride())
+
+    def dim(self):
+        return len(self.shape)
+
+    def stride(self, i):
+        return self._stride[i]
+
+    def data_ptr(self):
+        return 1 << 20
+
+    def is_contiguous(self):
+        return self._stride == tuple(torch.empty(self.shape, device="meta").stride())
+
+
+class _NoLaunch:
+    """libmi_attn whose weight gradient suits every size and may not be launched."""
+
+    def mi_wgrad_suits(self, *sizes):
+        return 1
+
+    def mi_wgrad_workspace(self, *sizes):
+        raise AssertionError(f"about to launch with {sizes}")
+
+
+@pytest.mark.parametrize("dy,x,dw", [
+    (_OnGpu(512, 136), _OnGpu(256, 64), None),            # fewer rows than dy
+    (_OnGpu(512, 136), _OnGpu(1024, 64), None),
+    (_OnGpu(512, 136), _OnGpu(512, 64), _OnGpu(128, 64)),  # a gradient of other sizes
+    (_OnGpu(512, 136), _OnGpu(512, 64), _OnGpu(136, 32)),
+    (_OnGpu(512, 136), _OnGpu(512, 64), _OnGpu(136 * 64)),
+    (_OnGpu(512, 136), _OnGpu(512, 64), _OnGpu(136, 64, stride=(128, 1))),
+    (_OnGpu(512, 136), _OnGpu(512, 64), _OnGpu(136, 64, stride=(1, 136))),
+    (_OnGpu(2, 256, 136), _OnGpu(512, 64), None),
+])
+def test_wgrad_takes_only_operands_that_fit(monkeypatch, dy, x, dw):
+    """The kernel indexes by dy's rows and dweight [out, in]: other operands are
+    left to the general product, which refuses them."""
+    monkeypatch.setattr(_lib, "lib", lambda: _NoLaunch())
+    assert _lib.wgrad(dy, x, dw) is None
+
+
+def test_wgrad_operands_that_fit(monkeypatch):
+    monkeypatch.setattr(_lib, "lib", lambda: _NoLaunch())
+    with pytest.raises(AssertionError, match="about to launch"):
+        _lib.wgrad(_OnGpu(512, 136), _OnGpu(512, 64), _OnGpu(136, 64))
