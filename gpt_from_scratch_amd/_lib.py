@@ -366,9 +366,26 @@ def rmsnorm_workspace(rows: int, hidden: int) -> int:
     return int(lib().mi_rmsnorm_bwd_workspace(rows, hidden))
 
 
+def _check_norm_bwd(x, weight, rstd, dy):
+    """What the backward indexes by x's shape, and reads in the dtypes of x and
+    the weight: y's gradient, the weight and the dense fp32 rstd."""
+    want = torch.float32 if weight.dtype == torch.float32 else x.dtype
+    if dy.shape != x.shape or dy.dtype != want:
+        raise ValueError(f"the gradient must match x ({tuple(x.shape)}, {want}); got "
+                         f"{tuple(dy.shape)}, {dy.dtype}")
+    if weight.shape != x.shape[-1:] or not weight.is_contiguous():
+        raise ValueError(f"weight must be a contiguous [{x.shape[-1]}] tensor; got "
+                         f"{tuple(weight.shape)} / {weight.stride()}")
+    if rstd.dtype != torch.float32 or rstd.numel() * x.shape[-1] != x.numel() \
+            or not rstd.is_contiguous():
+        raise ValueError(f"rstd must be a contiguous float32 tensor, one value per row of "
+                         f"{tuple(x.shape)}; got {rstd.dtype} {tuple(rstd.shape)}")
+
+
 def rmsnorm_bwd(x, weight, rstd, dy, dx, dweight, workspace, accumulate=False):
     """Enqueue the RMSNorm backward: dx (x's shape and dtype), dweight [hidden]
     (added to its contents with `accumulate`)."""
+    _check_norm_bwd(x, weight, rstd, dy)
     _require_gpu(x, weight, rstd, dy, dx, dweight, workspace)
     rows, xs = _rows(x)
     _, dys = _rows(dy)
@@ -399,6 +416,7 @@ def rmsnorm_add_bwd(sum_in, weight, rstd, dy, dsum, dx, dweight, workspace, accu
     """Enqueue the backward of rmsnorm_add_fwd: dx = norm backward over sum_in
     plus dsum (the gradient of x and of res), dweight [hidden] (added to its
     contents with `accumulate`)."""
+    _check_norm_bwd(sum_in, weight, rstd, dy)
     _require_gpu(sum_in, weight, rstd, dy, dsum, dx, dweight, workspace)
     rows, xs = _rows(sum_in)
     _, dys = _rows(dy)

@@ -443,7 +443,9 @@ Tensor norm_bwd(const Tensor& x, const Tensor& w, const Tensor& rstd, const Tens
   const int64_t H = x.size(-1), n = rstd.numel();
   dense("rstd", rstd, x.sizes().slice(0, x.dim() - 1), at::kFloat, dy);
   dense("weight", w, {H}, w.scalar_type(), dy);
-  strided("saved x", x, dy.sizes(), x.scalar_type(), dy);
+  // dy is read in the dtype that x and the weight gave y
+  strided("the gradient", dy, x.sizes(),
+          w.scalar_type() == at::kFloat ? at::kFloat : x.scalar_type(), x);
   const int64_t nws = lib.mi_rmsnorm_bwd_workspace(n, H);
   Tensor ws = empty_f32({nws}, x);
   const Tensor g = grad_into ? grad_target(w, weight_dtype) : Tensor();

@@ -185,6 +185,22 @@ def test_hooks_that_change_a_saved_tensor_are_refused(gpu):
                     sum(o.sum() for o in outs).backward()
 
 
+def test_hooks_that_change_the_norms_dtypes_are_refused(gpu):
+    """The gradient is read in the dtype that the saved x and weight stand for."""
+    import gpt_from_scratch_amd as fw
+    x, r, w = _t(1, 40, 64), _t(2, 40, 64), _t(3, 64)
+    norms = [(f, [x, w]) for f in (fw.rms_norm, fw.FusedRMSNorm.apply)] + \
+            [(f, [x, r, w]) for f in (fw.add_rms_norm, fw.FusedAddRMSNorm.apply)]
+    for fn, tensors in norms:
+        for which in (lambda t: t.dim() == 1, lambda t: True):  # the weight alone, and x too
+            xs = [_leaf(t, True) for t in tensors]
+            with torch.autograd.graph.saved_tensors_hooks(
+                    lambda t: t, lambda t: t.float() if which(t) else t):
+                outs = _outs(fn(*xs, 1e-5))
+                with pytest.raises(ValueError):
+                    sum(o.sum() for o in outs).backward()
+
+
 def test_gradient_added_into_the_weights(gpu):
     import gpt_from_scratch_amd as fw
     from gpt_from_scratch_amd.harness import gpt

@@ -59,3 +59,22 @@ def test_wgrad_operands_that_fit(monkeypatch):
     monkeypatch.setattr(_lib, "lib", lambda: _NoLaunch())
     with pytest.raises(AssertionError, match="about to launch"):
         _lib.wgrad(_OnGpu(512, 136), _OnGpu(512, 64), _OnGpu(136, 64))
+
+
+@pytest.mark.parametrize("x,w,rstd,dy", [
+    ((6, 64, "bf"), (64, "f"), 6, (6, 64, "bf")),    # y was fp32: so is its gradient
+    ((6, 64, "f"), (64, "f"), 6, (6, 64, "bf")),
+    ((6, 64, "bf"), (64, "bf"), 6, (6, 64, "f")),
+    ((6, 64, "bf"), (64, "bf"), 6, (5, 64, "bf")),
+    ((6, 64, "bf"), (32, "bf"), 6, (6, 64, "bf")),
+    ((6, 64, "bf"), (64, "bf"), 5, (6, 64, "bf")),
+])
+def test_norm_backward_takes_only_operands_that_fit(x, w, rstd, dy):
+    """Refused by shape and dtype, before the device is looked at."""
+    t = lambda s: torch.zeros(s[:-1], dtype={"f": torch.float32, "bf": torch.bfloat16}[s[-1]])
+    x, w, dy, rstd = t(x), t(w), t(dy), torch.zeros(rstd)
+    ws = torch.zeros(64)
+    with pytest.raises(ValueError):
+        _lib.rmsnorm_bwd(x, w, rstd, dy, x, w, ws)
+    with pytest.raises(ValueError):
+        _lib.rmsnorm_add_bwd(x, w, rstd, dy, x, x, w, ws)
