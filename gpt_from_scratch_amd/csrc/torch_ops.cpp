@@ -302,7 +302,7 @@ struct RoPEQK : torch::autograd::Function<RoPEQK> {
 // Strides of a [S, B, ..., H, D] tensor's slice in the kernels' [B, H, S, D] order.
 struct BHSD {
   int64_t s[4];
-  BHSD(int64_t S, int64_t B, int64_t H) : s{B, H, S, 1} {}
+  BHSD(int64_t S, int64_t B, int64_t H, int64_t D = 1) : s{B, H, S, D} {}
 };
 
 struct Block : torch::autograd::Function<Block> {
@@ -352,7 +352,10 @@ struct Block : torch::autograd::Function<Block> {
     go = go.view(shape);
     if (go.stride(-1) != 1 || !rows16(go)) go = go.contiguous();
     Tensor dqkv = empty({S, B, 3 * H * D}, qkv), ws = empty_f32({2, B, H, S}, qkv);
-    const BHSD rs(B * 2 * H * D, 2 * H * D, D), vs(x.stride(0), x.stride(1), x.stride(3)),
+    // the saved qkv may have come back in another layout: its own strides, which
+    // the C ABI checks
+    const BHSD rs(B * 2 * H * D, 2 * H * D, D),
+        vs(x.stride(0), x.stride(1), x.stride(3), x.stride(4)),
         os(B * H * D, H * D, D), gs(go.stride(0), go.stride(1), go.stride(2)),
         ds(B * 3 * H * D, 3 * H * D, D);
     char *rp = (char*)rot.data_ptr(), *dp = (char*)dqkv.data_ptr();

@@ -185,6 +185,27 @@ def test_hooks_that_change_a_saved_tensor_are_refused(gpu):
                     sum(o.sum() for o in outs).backward()
 
 
+def test_hooks_that_change_a_saved_layout(gpu):
+    """The same values in other strides: the same gradients, or refused."""
+    turned = lambda t: t.transpose(0, -1).contiguous().transpose(0, -1) if t.dim() > 1 else t
+    refused = 0
+    for name, (fn, cls, tensors, args) in _cases().items():
+        grads = []
+        for hook in (lambda t: t, turned):
+            xs = [_leaf(t, True) for t in tensors]
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t, hook):
+                outs = _outs(fn(*xs, *args))
+                try:
+                    sum(o.sum() for o in outs).backward()
+                except Exception as e:
+                    assert type(e).__name__ in ("ValueError", "RuntimeError", "MiError"), name
+                    refused += 1
+                    continue
+            grads.append([x.grad for x in xs])
+        assert len(grads) == 1 or all(torch.equal(a, b) for a, b in zip(*grads)), name
+    assert refused
+
+
 def test_hooks_that_change_the_norms_dtypes_are_refused(gpu):
     """The gradient is read in the dtype that the saved x and weight stand for."""
     import gpt_from_scratch_amd as fw
