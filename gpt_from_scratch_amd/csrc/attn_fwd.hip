@@ -296,7 +296,10 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
     mx = max_halves(mx) * c;
     if (__any(mx > m_run + kRescaleSlack)) {
       const float m_new = fmaxf(m_run, mx);
-      const float alpha = fast_exp2(m_run - m_new);
+      // KS = 2: a row that has scored -inf alone in this wave's part of the tiles
+      // is rescaled with the wave's other rows: by 2^(-inf - 0) = 0, not by NaN
+      const float ref = KS > 1 && m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = fast_exp2(m_run - ref);
       l_run *= alpha;
 #pragma unroll
       for (int db = 0; db < C::DB; ++db) acc[db] *= alpha;
@@ -356,8 +359,8 @@ __global__ __launch_bounds__(256, FwdCfg<D>::WAVES_PER_EU) void attn_fwd_mfma_ke
       // recompute S from the staged K tile and take the exact step.  D = 128
       // takes the exact step every time (the skip's extra code spills there).
       float psum = 0.f;
-      // (KS = 2: a wave's part of the tiles so far may have held -inf scores
-      // alone; it has no reference yet, and takes P = 0 for them)
+      // (KS = 2: a row's scores in the wave's part of the tiles so far may have
+      // been -inf alone; such a row has no reference yet, and takes P = 0 for them)
       bool exact = D != 64 || j == 0;
       if constexpr (KS > 1) exact = exact || __any(m_run == -INFINITY);
       if (!exact) {

@@ -90,3 +90,29 @@ def test_scores_of_minus_infinity(gpu, D, H):
     z = q[..., 1:].float() @ k[:, :, keep, 1:].float().transpose(-1, -2).contiguous() / D ** 0.5
     assert_close_bf16("o", o, z.softmax(-1) @ v[:, :, keep].float())
     assert_close_bf16("lse", lse, z.logsumexp(-1))
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("H", [2, 600])
+def test_some_rows_score_minus_infinity(gpu, D, H, causal):
+    """Single query rows whose products with one 32-key block overflow to -inf
+    (finite inputs), beside rows that score it normally: the block has no part in
+    those rows, and every row is right.  The block is all that one of two waves
+    that share a row has seen of it when its other rows find their maximum."""
+    S = 160
+    q, k, v = (seeded((1, 2, S, D), 60 + i).to(gpu).repeat(1, H // 2, 1, 1) for i in range(3))
+    q[..., 0], k[..., 0] = 0.0, 0.0
+    rows = [67, 96, 127, 140]
+    q[:, :, rows, 0] = 2.0 ** 127
+    from gpt_from_scratch_amd import flash_attn_forward
+    for first in (0, 32, 64):
+        kb = k.clone()
+        kb[:, :, first:first + 32, 0] = -256.0
+        o, lse = flash_attn_forward(q, kb, v, causal)
+        z = q[:, :2].double() @ kb[:, :2].double().transpose(-1, -2).contiguous() / D ** 0.5
+        if causal:
+            z = z.masked_fill(torch.ones(S, S, dtype=torch.bool, device=gpu).triu(1), -float("inf"))
+        reps = (1, H // 2, 1, 1)
+        assert_close_bf16("o", o, (z.softmax(-1) @ v[:, :2].double()).repeat(*reps))
+        assert_close_bf16("lse", lse, z.logsumexp(-1).repeat(*reps[:3]))
