@@ -31,11 +31,11 @@
 // feeds four 32-cycle products, a quarter of the LDS bandwidth, so 16 rows per
 // wave are enough; the softmax is 16 exponentials per 128 products at D = 64.
 // Reached, causal, products executed (the backward's recomputed ones counted):
-// B4 H16 S2048 D64 forward 314 us (110 TFLOP/s), backward 985 us (122); on the
+// B4 H16 S2048 D64 forward 301 us (115 TFLOP/s), backward 1017 us (118); on the
 // vector ALUs these took 1357 and 5500 us, B2 H12 S1000 D64 216 and 774 us (now
-// 42 and 123) and B1 H12 S256 D64 38 and 105 us (10 and 17).  Errors against
-// float64 are no larger (B2 H12 S1000: O 2.8e-7 against 3.3e-7, dK 8.0e-7
-// against 7.9e-7).
+// 42 and 129) and B1 H12 S256 D64 38 and 105 us (8.5 and 17).  Errors against
+// float64 are no larger than the vector kernels' (partial_sums); with one sum per
+// product they were, and these took 298 and 979, 40 and 120, 8.5 and 16.6 us.
 #include <type_traits>
 
 #include "mi_device.h"
@@ -56,6 +56,10 @@ struct Cfg {
   static constexpr int KB = D / 16;                       // 16-column blocks
   static constexpr int W = KB >= 4 ? 4 : KB;              // adjacent columns per lane
   static constexpr int NH = KB / W;                       // 16 W-column spans
+  // Partial sums of a score and of a dO V^T product.  Scores have the same in
+  // both directions, so that the backward's P repeats the forward's rounding.
+  static constexpr int NPS = D == 16 ? 2 : D == 128 ? 8 : 4;
+  static constexpr int NPD = D == 16 ? 2 : 8;
 };
 
 // Chunk swizzle of a row: 16 rows of one chunk column, and the chunks of one
@@ -145,20 +149,37 @@ __device__ __forceinline__ void load_resident(const float* p, int64_t ss, int ro
   for (int s = 0; s < Cfg<D>::KB; ++s) f[s] = load4<VEC>(p + row * ss + 16 * s + 4 * g);
 }
 
-// (rows 16 b .. of the tile) x (resident rows), over the head dim.
-template <int D>
+// (rows 16 b .. of the tile) x (resident rows), over the head dim: NP partial
+// sums of D / NP products each, added by halves.  One chain of D products
+// rounds more: errors against float64 at S = 48, D = 128, causal, were 1.7 (O)
+// and 1.6 (dQ) times those of the vector kernels, whose eight lanes' chains are
+// added by halves too; with Cfg's partial sums they are 0.89 and 0.99 times.
+// The scheduling barrier keeps one partial sum's products in flight at a time:
+// all of them interleaved need up to 90 more registers (50 to 70 bytes of scratch
+// at D = 64 and 128) and ran no faster.
+template <int D, int NP, int LO = 0, int HI = NP>
+__device__ __forceinline__ f32x4 partial_sums(const f32x4 (&x)[Cfg<D>::KB],
+                                              const f32x4 (&f)[Cfg<D>::KB]) {
+  if constexpr (HI - LO > 1) {
+    const f32x4 lo = partial_sums<D, NP, LO, (LO + HI) / 2>(x, f);
+    __builtin_amdgcn_sched_barrier(0);
+    return lo + partial_sums<D, NP, (LO + HI) / 2, HI>(x, f);
+  } else {
+    constexpr int N = D / 4 / NP;  // four products each
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = N * LO; e < N * HI; ++e) acc = mfma4(x[e / 4][e % 4], f[e / 4][e % 4], acc);
+    return acc;
+  }
+}
+template <int D, int NP>
 __device__ __forceinline__ f32x4 row_product(const float* tile, int b, int i, int g,
                                              const f32x4 (&f)[Cfg<D>::KB]) {
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   f32x4 x[Cfg<D>::KB];
 #pragma unroll
   for (int s = 0; s < Cfg<D>::KB; ++s)
     x[s] = *(const f32x4*)(tile + (16 * b + i) * D + 4 * ((4 * s + g) ^ f32_swz<D>(i)));
-#pragma unroll
-  for (int s = 0; s < Cfg<D>::KB; ++s)
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) acc = mfma4(x[s][jj], f[s][jj], acc);
-  return acc;
+  return partial_sums<D, NP>(x, f);
 }
 
 // acc += (rows 16 b .. of the tile, transposed) x p, p in accumulator form.
@@ -263,7 +284,7 @@ __global__ __launch_bounds__(NT, 2) void attn_fwd_f32_kernel(AttnArgs a, int n_t
     for (int n = 0; n < NB; ++n) {
       const int blk = slice + KS * n, kb = kv0 + 16 * blk;
       if (MASKED && kb > last) continue;
-      st[n] = row_product<D>(Kt, blk, io, go, qf);
+      st[n] = row_product<D, C::NPS>(Kt, blk, io, go, qf);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int key = kb + 4 * g + r;
@@ -435,8 +456,8 @@ __device__ __forceinline__ void bwd_item(const AttnArgs& a, int bh, int r0, floa
       int io = i, go = g;
       opaque(io);
       opaque(go);
-      f32x4 p = row_product<D>(T0, blk, io, go, f0);
-      f32x4 ds = row_product<D>(T1, blk, io, go, f1);
+      f32x4 p = row_product<D, C::NPS>(T0, blk, io, go, f0);
+      f32x4 ds = row_product<D, C::NPD>(T1, blk, io, go, f1);
       f32x4 el = {lse2, lse2, lse2, lse2}, ed = {dl, dl, dl, dl};
       if constexpr (DKDV) {
         el = *(const f32x4*)&stat[0][16 * blk + 4 * g];
@@ -492,9 +513,11 @@ __device__ __forceinline__ void bwd_item(const AttnArgs& a, int bh, int r0, floa
 // dK/dV and dQ items in one launch, each kind's longest first and the longer
 // kind (four products against three) before the other; `kinds` = 1 runs the
 // dK/dV items alone, 2 the dQ items alone.
+// D = 64 asks for three waves per SIMD: left to itself, the compiler takes more
+// registers than those leave at KS = 2 (B1 H12 S1000, not causal: 150 us, not 120).
 template <int D, int KS, bool VEC>
-__global__ __launch_bounds__(NT, 2) void attn_bwd_f32_kernel(AttnArgs a, int n_tiles, int kinds,
-                                                             int n_cu) {
+__global__ __launch_bounds__(NT, D == 64 ? 3 : 2) void attn_bwd_f32_kernel(AttnArgs a, int n_tiles,
+                                                                           int kinds, int n_cu) {
   __shared__ __attribute__((aligned(16))) float T0[TR * D];
   __shared__ __attribute__((aligned(16))) float T1[TR * D];
   __shared__ __attribute__((aligned(16))) float stat[2][TR];
@@ -535,10 +558,11 @@ hipError_t launch_bwd(const AttnArgs& a, int kinds, hipStream_t st) {
 // fill the chip and shorten the longest chain.  By the number of 64-row
 // workgroups (the backward has two kinds of them in one launch, so its lines
 // lie at half the count), causal, KS = 4 / 2 / 1 in us:
-//   48 (B1 H12 S256 D64):   forward 10.2 / 10.5 / 15.1, backward 16.7 / 19.7 / 28.7
-//   192 (B1 H12 S1000 D64): forward 27.0 / 34.0 / 49.7, backward 74 / 71 / 107
-//   384 (B2 H12 S1000 D64): forward 50.4 / 42.0 / 58.9, backward 131 / 123 / 126
-//   2048 (B4 H16 S2048 D64): forward 432 / 332 / 314, backward 1205 / 1046 / 985
+//   48 (B1 H12 S256 D64):    forward 8.5 / 11.1 / 15.1, backward 17.4 / 20.4 / 30.0
+//   192 (B1 H12 S1000 D64):  forward 28.5 / 36.3 / 50.7, backward 79 / 75 / 111
+//   384 (B2 H12 S1000 D64):  forward 43.7 / 40.7 / 57.5, backward 128 / 127 / 129
+//   768 (B4 H12 S1000 D64):  forward 79 / 76 / 67, backward 247 / 222 / 221
+//   2048 (B4 H16 S2048 D64): forward 384 / 336 / 300, backward 1215 / 1071 / 1016
 // The gradient stages run alone (`kinds` 1 or 2) split as they do together,
 // so that their sums have the same order.
 int row_split(const AttnArgs& a, int line) {

@@ -169,3 +169,59 @@ def test_fp32_masked_and_infinite_scores(gpu, B, H):
     assert torch.allclose(lse[:, :, rows].double(), z.logsumexp(-1)[:, :, rows], atol=2e-5)
     assert torch.allclose(o[:, :, rows].double(), (p @ v[:, :, :40].double())[:, :, rows],
                           atol=2e-5)
+
+
+def _lane_chains(q, k, v, do, causal):
+    """o, dq, dk, dv in fp32 as vector kernels sum them: a score is 8 lanes' (4 at
+    D = 16) chains of multiply-adds over their 4-float chunks, added by halves; sums
+    over keys and queries are chains."""
+    fma = lambda a, b, c: (a.double() * b.double() + c.double()).float()
+    B, H, S, D = q.shape
+
+    def rows(a, b):  # [.., S, S]
+        lanes = 8 if D >= 32 else 4
+        t = [torch.zeros(B, H, S, S, device=q.device) for _ in range(lanes)]
+        for d in range(D):
+            p = d // 4 % lanes
+            t[p] = fma(a[..., d].unsqueeze(-1), b[..., d].unsqueeze(-2), t[p])
+        while len(t) > 1:
+            t = [x + y for x, y in zip(t[::2], t[1::2])]
+        return t[0]
+
+    def cols(w, x):  # sum over j of w[.., i, j] x[.., j, :], one chain
+        t = torch.zeros_like(x)
+        for j in range(S):
+            t = fma(w[..., j].unsqueeze(-1), x[..., j, :].unsqueeze(-2), t)
+        return t
+
+    c = torch.tensor(math.log2(math.e) / math.sqrt(D), device=q.device)
+    z = rows(q, k)
+    if causal:
+        z = z.masked_fill(torch.ones(S, S, dtype=torch.bool, device=q.device).triu(1), -math.inf)
+    m = (z * c).amax(-1, keepdim=True)
+    p = (z * c - m).exp2()
+    l = torch.zeros_like(m)
+    for j in range(S):
+        l = l + p[..., j:j + 1]
+    o = cols(p, v) * (1 / l)
+    lse = (m + l.log2()) * math.log(2)  # as it is kept between the passes
+    p = fma(z, c, -(lse * math.log2(math.e))).exp2()
+    ds = p * (rows(do, v) - (do * o).sum(-1, keepdim=True))
+    T = lambda t: t.transpose(-1, -2)
+    scale = 1 / math.sqrt(D)
+    return o, cols(ds, k) * scale, cols(T(ds), q) * scale, cols(T(p), do)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("S", [48, 65, 160])
+def test_fp32_errors_are_no_larger_than_lane_chains(gpu, S, D, causal):
+    """The matrix cores' sums against float64 are no further off than the vector
+    kernels' order (5% for the sample: 24 heads, 2-norm)."""
+    q, k, v, do = _inputs(2, 12, S, D, 17 * S + D, gpu)
+    o, _, *grads = _run(q, k, v, do, causal, _dense)
+    want = (attention_forward(q, k, v, causal)[0], *attention_backward(q, k, v, do, causal)[:3])
+    for name, got, ref, w in zip(("o", "dq", "dk", "dv"), (o, *grads),
+                                 _lane_chains(q, k, v, do, causal), want):
+        e, most = (float((t.double() - w.double()).norm() / w.double().norm()) for t in (got, ref))
+        assert e <= 1.05 * most, f"{name}: error {e:.3g} against {most:.3g}"
