@@ -1,7 +1,7 @@
 """Compiler resource report of the gfx950 kernels (CPU only: hipcc cross-compiles).
 
-The attention kernels (matrix-core and exact-fp32), RoPE and the model
-operators must not use scratch memory (register spills or run-time-indexed
+The attention kernels (matrix-core and exact-fp32), RoPE, the weight gradient
+and the model operators must not use scratch memory (register spills or run-time-indexed
 private arrays), and the hot attention kernels must keep the occupancy their
 tiling assumes.  The one documented exception is the causal combined backward
 at head dims 16 and 32 for sequence lengths that are not a multiple of 64 (36
@@ -19,7 +19,8 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "gpt_from_scratch_amd", "csrc")
 HIPCC = "/opt/rocm/bin/hipcc"
-SOURCES = ("attn_fwd.hip", "attn_bwd.hip", "attn_valu.hip", "rope.hip", "model_ops.hip")
+SOURCES = ("attn_fwd.hip", "attn_bwd.hip", "attn_f32.hip", "attn_valu.hip", "rope.hip",
+           "model_ops.hip", "wgrad.hip")
 # the causal combined backward at head dims 16 and 32 for sequence lengths
 # that are not a multiple of 64 (36 bytes per lane: scalar registers spilled)
 ALLOWED_SCRATCH = re.compile(r"attn_bwd_kernel<mi::(BF16|F16), 64, true, (true|false), "
