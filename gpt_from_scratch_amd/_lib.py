@@ -309,14 +309,16 @@ def rope_qk(q, k, cos, sin, q_out, k_out, inverse: bool):
 
 def _rows(t: torch.Tensor):
     """(rows, row stride) of t viewed as rows over its last dim (unit stride)."""
-    if t.stride(-1) != 1:
-        raise ValueError("the vocabulary dim must have unit stride")
     lead = t.shape[:-1]
     rows = 1
     for n in lead:
         rows *= n
-    if t.dim() == 1:
-        return 1, t.shape[-1]
+    # the strides of a contiguous tensor's size-1 dims mean nothing (a transposed
+    # [1, S, H] keeps S * H there): its rows lie one behind the other
+    if t.is_contiguous():
+        return rows, t.shape[-1]
+    if t.stride(-1) != 1:
+        raise ValueError("the vocabulary dim must have unit stride")
     # the leading dims must collapse into one row index with a single stride
     rs = t.stride(-2)
     expect = rs

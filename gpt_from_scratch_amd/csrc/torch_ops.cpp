@@ -113,14 +113,15 @@ Tensor empty_f32(at::IntArrayRef sizes, const Tensor& like) {
 }
 
 // Rows over the last dim as the C ABI takes them: count and stride; nothing if
-// the leading dims are not one row axis or rows overlap.
+// the leading dims are not one row axis or rows overlap.  The strides of a
+// contiguous tensor's size-1 dims mean nothing: its rows lie one behind the other.
 struct Rows {
   int64_t n, stride;
 };
 std::optional<Rows> rows_of(const Tensor& t) {
   const int64_t d = t.dim(), h = t.size(-1);
+  if (t.is_contiguous()) return Rows{h ? t.numel() / h : 0, h};
   if (t.stride(-1) != 1) return std::nullopt;
-  if (d == 1) return Rows{1, h};
   const int64_t rs = t.stride(-2);
   int64_t n = 1, expect = rs;
   for (int64_t i = d - 2; i >= 0; --i) {
@@ -138,8 +139,6 @@ Rows rows(const Tensor& t) {
                     t.sizes(), " / ", t.strides());
   return *r;
 }
-// Whether as_rows gives rows (a size-1 last dim may keep another stride).
-bool has_rows(const Tensor& t) { return rows_of(t) || t.size(-1) > 1; }
 
 // A tensor that a backward indexes as dense: what was saved may come back
 // through a saved-tensor hook as something else.
@@ -430,7 +429,7 @@ Tensor grad_target(const Tensor& w, at::ScalarType weight_dtype) {
 
 bool norm_ok(const Tensor& x, const Tensor& w) {
   return x.dim() >= 1 && w.dim() == 1 && x.size(-1) == w.size(0) && code(x) >= 0 && code(w) >= 0 &&
-         one_device(x, w) && has_rows(x);
+         one_device(x, w);
 }
 
 Tensor norm_out(const Tensor& x, const Tensor& w) {
@@ -717,7 +716,6 @@ PyObject* py_xent(PyObject*, Args a, Py_ssize_t n) {
   Tensor z, t;
   PLAIN(n == 2 && plain(a[0], z) && plain(a[1], t) && plain_context() && z.dim() >= 1 &&
         t.sizes() == z.sizes().slice(0, z.dim() - 1) && code(z) >= 0 && one_device(z, t) &&
-        has_rows(z) &&
         (t.scalar_type() == at::kLong || t.scalar_type() == at::kInt ||
          t.scalar_type() == at::kShort || t.scalar_type() == at::kByte ||
          t.scalar_type() == at::kChar));
@@ -743,7 +741,7 @@ PyObject* py_add_rms_norm(PyObject*, Args a, Py_ssize_t n) {
   bool into;
   PLAIN(n == 5 && plain(a[0], x) && plain(a[1], res) && plain(a[2], w) && plain_context() &&
         norm_ok(x, w) && res.sizes() == x.sizes() && res.scalar_type() == x.scalar_type() &&
-        one_device(x, res) && has_rows(res) && number(a[3], eps) && truth(a[4], into));
+        one_device(x, res) && number(a[3], eps) && truth(a[4], into));
   const variable_list r = released([&] { return AddRMSNorm::apply(x, res, w, eps, into); });
   return pair(r[0], r[1]);
   END_HANDLE_TH_ERRORS
@@ -753,7 +751,7 @@ PyObject* py_swiglu(PyObject*, Args a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Tensor gu;
   PLAIN(n == 1 && plain(a[0], gu) && plain_context() && gu.dim() >= 1 && gu.size(-1) % 2 == 0 &&
-        code(gu) >= 0 && has_rows(gu));
+        code(gu) >= 0);
   return THPVariable_Wrap(released([&] { return SwiGLU::apply(gu); }));
   END_HANDLE_TH_ERRORS
 }

@@ -112,3 +112,30 @@ def test_linear_grad_into_falls_back_without_buffer(gpu):
     first = w.grad.clone()
     _linear_into_grad(x.detach(), w).backward(gy)  # accumulated into the existing grad
     torch.testing.assert_close(w.grad.float(), 2 * first.float(), rtol=2 ** -7, atol=1e-2)
+
+
+def test_batch_of_one(gpu):
+    """One sequence, whose [S, 1, H] activations have a size-1 dim of any stride:
+    the logits, losses and gradients of the same sequence in a batch of two.  A
+    product's kernel may depend on its row count, so the two may round differently:
+    2%, twice what one to three such layers in bf16 are off float64 (0.9%)."""
+    from gpt_from_scratch_amd import vocab_parallel_cross_entropy
+    from gpt_from_scratch_amd.harness import GPT
+    torch.manual_seed(0)
+    S = 100
+    cfg = GPTConfig(vocab_size=1000, hidden_size=256, num_layers=2, num_attention_heads=4,
+                    max_position_embeddings=S, intermediate_size=512)
+    ids = torch.randint(0, 1000, (1, S + 1), device=gpu)
+    for fuse in (True, False):
+        model = GPT(cfg, gpu, fuse_add_norm=fuse).to(torch.bfloat16)
+        out = []
+        for n in (1, 2):
+            x = ids.repeat(n, 1)
+            model.zero_grad()
+            z = model(x[:, :-1].contiguous())
+            loss = vocab_parallel_cross_entropy(z, x[:, 1:].t().contiguous())
+            loss.float().mean().backward()
+            out.append([z[:, :1], loss[:, :1]] + [p.grad for p in model.parameters()])
+        for a, b in zip(*out):
+            a, b = a.detach().double(), b.detach().double()
+            assert float((a - b).norm() / b.norm()) < 0.02

@@ -81,6 +81,16 @@ def _cases():
         c[f"norm-strided-{dt}"] = (fw.rms_norm, fw.FusedRMSNorm.apply,
                                    [_t(n, 7, 4, 96, dtype=dt).transpose(0, 1), _t(3, 96, dtype=dt)],
                                    [1e-5, False])
+        turned = lambda *shape: _t(n, *shape, dtype=dt).transpose(0, 1)  # [S, 1, H]: odd strides
+        c[f"norm-batch-1-{dt}"] = (fw.rms_norm, fw.FusedRMSNorm.apply,
+                                   [turned(1, 7, 96), _t(3, 96, dtype=dt)], [1e-5, False])
+        c[f"add_norm-batch-1-{dt}"] = (fw.add_rms_norm, fw.FusedAddRMSNorm.apply,
+                                       [turned(1, 7, 96), _t(4, 7, 1, 96, dtype=dt),
+                                        _t(3, 96, dtype=dt)], [1e-5, False])
+        c[f"swiglu-batch-1-{dt}"] = (fw.swiglu, fw.SwiGLU.apply, [turned(1, 7, 96)], [])
+        c[f"xent-batch-1-{dt}"] = (fw.vocab_parallel_cross_entropy,
+                                   fw.VocabParallelCrossEntropy.apply, [turned(1, 6, 201)],
+                                   [tgt[:, :1]])
         c[f"swiglu-{dt}"] = (fw.swiglu, fw.SwiGLU.apply, [_t(n, 3, 5, 2 * 72, dtype=dt)], [])
         c[f"swiglu-wide-{dt}"] = (fw.swiglu, fw.SwiGLU.apply, [_wide(_t(n, 15, 2 * 7, dtype=dt), 5)],
                                   [])

@@ -78,3 +78,24 @@ def test_norm_backward_takes_only_operands_that_fit(x, w, rstd, dy):
         _lib.rmsnorm_bwd(x, w, rstd, dy, x, w, ws)
     with pytest.raises(ValueError):
         _lib.rmsnorm_add_bwd(x, w, rstd, dy, x, x, w, ws)
+
+
+@pytest.mark.parametrize("t,want", [
+    (torch.zeros(1, 7, 8).transpose(0, 1).contiguous(), (7, 8)),   # strides (8, 56, 1)
+    (torch.zeros(1, 7, 8).transpose(0, 1), (7, 8)),
+    (torch.zeros(1, 1, 8).as_strided((1, 1, 8), (3, 5, 1)), (1, 8)),
+    (torch.zeros(6, 1).as_strided((6, 1), (1, 9)), (6, 1)),
+    (torch.zeros(8), (1, 8)),
+    (torch.zeros(5, 3, 8), (15, 8)),
+    (torch.zeros(5, 3, 11)[..., :8], (15, 11)),
+    (torch.zeros(5, 6, 8)[:, ::2], (15, 16)),
+])
+def test_rows_of_a_tensor(t, want):
+    assert _lib._rows(t) == want
+
+
+@pytest.mark.parametrize("t", [torch.zeros(3, 5, 8).transpose(0, 1), torch.zeros(1, 8).expand(4, 8),
+                               torch.zeros(4, 8)[:, ::2], torch.zeros(4, 7, 8)[:, :3]])
+def test_no_rows(t):
+    with pytest.raises(ValueError):
+        _lib._rows(t)
