@@ -26,6 +26,7 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TensorUtils.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -591,7 +592,9 @@ Tensor wgrad(const Tensor& dy, const Tensor& x, const Tensor& g) {
 
 struct LinearGradInto : torch::autograd::Function<LinearGradInto> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, bool into) {
-    ctx->save_for_backward({x, w});
+    // as F.linear, only what a gradient needs (and w where its .grad takes dw)
+    ctx->save_for_backward({w.requires_grad() ? x : Tensor(),
+                            x.requires_grad() || into ? w : Tensor()});
     ctx->saved_data["into"] = into;
     return at::linear(x, w);
   }
@@ -761,7 +764,9 @@ PyObject* py_linear_into_grad(PyObject*, Args a, Py_ssize_t n) {
   Tensor x, w;
   bool into;
   PLAIN(n == 3 && plain(a[0], x) && plain(a[1], w) && plain_context() && x.dim() >= 1 &&
-        w.dim() == 2 && x.size(-1) == w.size(1) && one_device(x, w) && truth(a[2], into));
+        w.dim() == 2 && x.size(-1) == w.size(1) && one_device(x, w) && truth(a[2], into) &&
+        !at::autocast::is_autocast_enabled(at::kCUDA) &&
+        (into || (x.scalar_type() == w.scalar_type() && (code(x) == MI_BF16 || code(x) == MI_F16))));
   return THPVariable_Wrap(released([&] { return LinearGradInto::apply(x, w, into); }));
   END_HANDLE_TH_ERRORS
 }

@@ -99,8 +99,13 @@ class _LinearGradInto(torch.autograd.Function):
 
 
 def _linear(x, w, into=False):
+    """``F.linear``, with `into` as _LinearGradInto; without, only the plain calls
+    that mi_wgrad may serve (16-bit GPU tensors, no autocast, transform or tangent)
+    leave torch's own operator."""
     y = _lib.ops().linear_into_grad(x, w, into) if x.is_cuda else None
-    return _LinearGradInto.apply(x, w, into) if y is None else y
+    if y is not None:
+        return y
+    return _LinearGradInto.apply(x, w, into) if into else F.linear(x, w)
 
 
 def _linear_into_grad(x, w):

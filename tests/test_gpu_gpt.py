@@ -139,3 +139,8 @@ def test_batch_of_one(gpu):
         for a, b in zip(*out):
             a, b = a.detach().double(), b.detach().double()
             assert float((a - b).norm() / b.norm()) < 0.02
+
+
+def test_linear_without_accumulation_is_torchs(gpu):
+    from test_harness import _linear_behaves_as_torchs
+    _linear_behaves_as_torchs("cuda")

@@ -94,3 +94,46 @@ def test_tiny_model_trains_on_cpu_with_eager_attention():
         losses.append(float(loss.detach()))
     assert abs(losses[0] - math.log(97)) < 0.5
     assert losses[-1] < losses[0]
+
+
+def _linear_behaves_as_torchs(dev):
+    """harness.gpt._linear (no accumulation into .grad) in the forms F.linear takes."""
+    from gpt_from_scratch_amd.harness.gpt import _linear
+    F = torch.nn.functional.linear
+    g = torch.Generator().manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=g).to(dev)
+
+    def passed(f, dtype, autocast, freeze=None, after=None):
+        x, w = (t.to(dtype, copy=True).requires_grad_() for t in (x0, w0))
+        if freeze == "x":
+            x.requires_grad_(False)
+        if freeze == "w":
+            w.requires_grad_(False)
+        with torch.autocast(torch.device(dev).type, torch.bfloat16, enabled=autocast):
+            y = f(x, w)
+        if after:  # the operand that no gradient needs may change before the backward
+            with torch.no_grad():
+                (w if freeze == "x" else x).add_(1)
+        (y.float().square().sum()).backward()
+        return [t for t in (y, x.grad, w.grad) if t is not None]
+
+    x0, w0 = r(4, 10, 24), r(16, 24)
+    for dtype, autocast, freeze, after in (
+            (torch.float32, True, None, False), (torch.float32, False, None, False),
+            (torch.bfloat16, True, None, False), (torch.bfloat16, False, None, False),
+            (torch.float32, True, "x", False), (torch.bfloat16, False, "x", True),
+            (torch.bfloat16, False, "w", True), (torch.float64, False, None, False)):
+        a, b = (passed(f, dtype, autocast, freeze, after) for f in (_linear, F))
+        assert len(a) == len(b) and all(p.dtype == q.dtype and torch.equal(p, q)
+                                        for p, q in zip(a, b)), (dtype, autocast, freeze)
+    for dtype in (torch.float32, torch.bfloat16):
+        x, w, t = x0.to(dtype), w0.to(dtype), r(4, 10, 24).to(dtype)
+        many = lambda f: torch.func.vmap(lambda u: f(u, w))(x)
+        tangent = lambda f: torch.func.jvp(lambda u: f(u, w), (x,), (t,))[1]
+        pull = lambda f: torch.func.grad(lambda u: f(x, u).float().square().sum())(w)
+        for form in (many, tangent, pull):
+            assert torch.equal(form(_linear), form(F))
+
+
+def test_linear_without_accumulation_is_torchs():
+    _linear_behaves_as_torchs("cpu")
