@@ -485,6 +485,8 @@ def wgrad(dy, x, dweight=None):
     st = lib().mi_wgrad(dtype_code(dy), rows, out, x.shape[1], _ptr(dy), dy.stride(0), _ptr(x),
                         x.stride(0), _ptr(dweight), int(acc), _ptr(ws), n, _stream(dy))
     _check(st, "mi_wgrad")
+    if acc:
+        torch.autograd.graph.increment_version(dweight)  # as addmm_ would
     return dweight
 
 

@@ -587,6 +587,7 @@ Tensor wgrad(const Tensor& dy, const Tensor& x, const Tensor& g) {
                      x.data_ptr(), x.stride(0), dw.data_ptr(), g.defined(), ws.data_ptr<float>(),
                      n, stream(dy)),
         "mi_wgrad");
+  if (g.defined()) g.unsafeGetTensorImpl()->bump_version();  // as addmm_ would
   return dw;
 }
 

@@ -95,6 +95,24 @@ def test_what_the_projection_hands_over(gpu):
     assert suits == [True, True, False, False]
 
 
+def test_a_gradient_that_a_graph_holds_is_known_to_have_changed(gpu):
+    """Accumulating into .grad counts as an in-place change of it, at sizes of
+    mi_wgrad as at others: a graph that saved it refuses its backward."""
+    from gpt_from_scratch_amd.harness import gpt
+    for M in (600, 200):  # mi_wgrad, addmm_
+        x, w, gy = seeded((M, 64), 1).to(gpu), seeded((136, 64), 2).to(gpu), seeded((M, 136), 3).to(gpu)
+        for fn in (gpt._linear, gpt._LinearGradInto.apply):
+            wl = w.clone().requires_grad_()
+            wl.grad = torch.ones_like(wl)
+            scale = torch.ones_like(wl).requires_grad_()
+            held = (wl.grad * scale).sum()
+            version = wl.grad._version
+            fn(x, wl, True).backward(gy)
+            assert wl.grad._version > version
+            with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+                held.backward()
+
+
 def test_operands_that_no_longer_fit_are_refused(gpu):
     """A saved x that a hook changed, or a gradient of other sizes: torch's
     products refuse them, as at sizes that mi_wgrad does not take, and the
