@@ -16,8 +16,6 @@
 // it can.  Reached with the sum: 690-760 TFLOP/s (8192 x 2304 x 768, 8192 x 768 x
 // 3072), 410 on 8192 x 768 x 768, whose partial tiles are 33 MB.  Tiles of 32
 // tokens (four workgroups per CU) took 45 and 75 us against 39 and 56.
-#include <algorithm>
-
 #include "mi_device.h"
 #include "mi_kernels.h"
 
@@ -191,26 +189,15 @@ int wgrad_splits(int64_t M, int64_t N, int64_t K) {
 }
 
 // Whether this beats the general GEMM library (addmm_ with beta = 1, which
-// splits no tokens at these sizes, and takes up to half as long again where M is
-// no multiple of 64).  us, library / this, bf16:
-//   M 8192:  768 x 768 (36 tiles) 49 / 24, 2304 x 768 (108) 65 / 39, 768 x 3072
-//            (144) 80 / 51, 4096 x 768 (192) 90.8 / 78.2, 6144 x 768 (288) 113 / 141
-//   M 2560:  768 x 768 19.2 / 16.7, 2304 x 768 24.6 / 23.2, 1024 x 1024 (64) 19.7 / 20.8
-//   M 2048:  768 x 768 16.5 / 15.4, 1536 x 512 (48) 16.6 / 16.6, 2304 x 768 20.3 / 23.2
-//   M 1536:  512 x 512 (16) 13.1 / 11.3, 2048 x 256 (32) 13.2 / 13.4, 768 x 768 13.3 / 14.0
-//   M 1500:  512 x 512 16.8 / 11.6, 768 x 768 17.0 / 13.8, 1536 x 512 17.1 / 15.3
-//   M 1024:  512 x 512 11.3 / 10.8, 768 x 768 11.4 / 12.4, 1000: 13.3 / 10.8, 13.3 / 12.3
-//   M 768:   512 x 512 9.5 / 12.3, 768 x 768 9.5 / 13.1: below 16 steps the tokens are
-//            not split
-//   M 400:   256 x 256 (4) 22.0 / 9.4, 128 x 64 (1) 10.0 / 9.3, 512 x 256 (8) 8.6 / 9.5:
-//            the library is slow at a few of the smallest weights
+// splits no tokens at these sizes).  us, library / this, bf16:
+//   M 8192:  768 x 768 48.0 / 23.3, 2304 x 768 63.3 / 39.9, 768 x 3072 79.5 / 56.9,
+//            4096 x 768 (192 tiles) 90.8 / 78.2, 6144 x 768 (288 tiles) 113 / 141
+//   M 3000:  2304 x 768 33.3 / 23.4          M 16384: 1024 x 1024 110 / 52
+//   M 2048:  2304 x 768 (108 tiles) 20.1 / 22.3, 1536 x 512 (48 tiles) 17.9 / 17.7
+//   M 256:   768 x 768 18.1 / 9.0
 bool wgrad_suits(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ((N + WT - 1) / WT) * ((K + WT - 1) / WT);
-  if (M < 256 || tiles > 192) return false;
-  if (tiles <= 4) return true;
-  if (M <= 15 * WM) return false;
-  if (M % 64) return tiles <= 48 || M >= 2560;
-  return M >= std::min<int64_t>(56 * tiles, 2560);
+  return M >= 256 && tiles <= 192 && (M >= 2560 || tiles <= 48);
 }
 
 hipError_t launch_wgrad(int dtype, WgradArgs a, hipStream_t st) {

@@ -99,16 +99,3 @@ def test_rows_of_a_tensor(t, want):
 def test_no_rows(t):
     with pytest.raises(ValueError):
         _lib._rows(t)
-
-
-@pytest.mark.parametrize("rows,out,inp,suits", [
-    (255, 128, 128, 0), (256, 128, 128, 1), (256, 256, 256, 1), (768, 512, 128, 1),  # 4 tiles
-    (768, 512, 256, 0), (960, 512, 256, 0), (961, 512, 256, 1), (1024, 512, 512, 1),
-    (1023, 768, 768, 1), (1024, 768, 768, 0), (1984, 768, 768, 0), (2048, 768, 768, 1),
-    (961, 1536, 512, 1), (960, 1536, 512, 0), (2496, 1536, 512, 0), (2560, 1536, 512, 1),
-    (2500, 1024, 1024, 0), (2561, 1024, 1024, 1), (2496, 2304, 768, 0), (2560, 2304, 768, 1),
-    (8192, 4096, 768, 1), (8192, 6144, 768, 0), (8191, 6144, 768, 0),
-])
-def test_wgrad_suits(rows, out, inp, suits):
-    """Both sides of each line of the choice between mi_wgrad and the general GEMM."""
-    assert _lib.lib().mi_wgrad_suits(rows, out, inp) == suits
