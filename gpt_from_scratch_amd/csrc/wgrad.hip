@@ -188,13 +188,22 @@ int wgrad_splits(int64_t M, int64_t N, int64_t K) {
   return (int)(s < 1 ? 1 : s);
 }
 
-// Whether this beats the general GEMM library (addmm_ with beta = 1, which
-// splits no tokens at these sizes).  us, library / this, bf16:
-//   M 8192:  768 x 768 48.0 / 23.3, 2304 x 768 63.3 / 39.9, 768 x 3072 79.5 / 56.9,
-//            4096 x 768 (192 tiles) 90.8 / 78.2, 6144 x 768 (288 tiles) 113 / 141
-//   M 3000:  2304 x 768 33.3 / 23.4          M 16384: 1024 x 1024 110 / 52
-//   M 2048:  2304 x 768 (108 tiles) 20.1 / 22.3, 1536 x 512 (48 tiles) 17.9 / 17.7
-//   M 256:   768 x 768 18.1 / 9.0
+// Whether this takes the place of the general GEMM library (addmm_ with beta = 1,
+// which splits no tokens at these sizes).  The kernels alone, us, library / this,
+// bf16 (weights of t tiles):
+//   M 8192:  768 x 768 (t 36) 49 / 24, 2304 x 768 (108) 65 / 39, 768 x 3072 (144)
+//            80 / 51, 4096 x 768 (192) 90.8 / 78.2, 6144 x 768 (288) 113 / 141
+//   M 3000:  2304 x 768 34 / 24              M 16384: 1024 x 1024 110 / 52
+//   M 2560:  2304 x 768 24.6 / 23.2, 1024 x 1024 (64) 19.7 / 20.8, 768 x 768 19.2 / 16.7
+//   M 2048:  2304 x 768 20.3 / 23.2, 1536 x 512 (48) 16.6 / 16.6, 768 x 768 16.5 / 15.4
+//   M 1500:  1536 x 512 17.1 / 15.3, 512 x 512 (16) 16.8 / 11.6
+//   M 1024:  1536 x 512 11.5 / 13.4, 512 x 512 11.3 / 10.8
+//   M 640:   768 x 768 8.8 / 12.0, 768 x 256 (12) 8.6 / 11.4, 256 x 256 (4) 24 / 11
+// Below 16 steps the tokens are not split, and there the library's kernel is the
+// shorter one but for the smallest weights.  The host bounds such a backward,
+// and it spends less on this launch than on torch's addmm_: forward and backward
+// of models of 4, 3 and 2 layers on 656, 600 and 726 tokens took 1.99, 1.51 and
+// 1.18 ms with this, 2.06, 1.59 and 1.20 with the library.
 bool wgrad_suits(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ((N + WT - 1) / WT) * ((K + WT - 1) / WT);
   return M >= 256 && tiles <= 192 && (M >= 2560 || tiles <= 48);

@@ -392,8 +392,8 @@ mi_status mi_swiglu_bwd(mi_dtype dtype, int64_t rows, int64_t inter, const void*
  * aligned and of a multiple of 8 elements; dweight dense.  workspace:
  * mi_wgrad_workspace(rows, out, in) floats, 16-byte aligned, contents
  * irrelevant.  mi_wgrad_suits: whether these sizes are ones it is built for
- * (long rows, few tiles of dweight); others are correct, but a general GEMM is
- * faster. */
+ * (256 rows or more, few tiles of dweight); others are correct, but a general
+ * GEMM is faster. */
 int mi_wgrad_suits(int64_t rows, int64_t out_features, int64_t in_features);
 int64_t mi_wgrad_workspace(int64_t rows, int64_t out_features, int64_t in_features);
 mi_status mi_wgrad(mi_dtype dtype, int64_t rows, int64_t out_features, int64_t in_features,
