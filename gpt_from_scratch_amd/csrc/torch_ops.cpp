@@ -6,14 +6,15 @@
 // the kernels of most calls take.  The functions below do the same work for a
 // plain call (measured, forward and backward, us: the attention block of a
 // GPT-2-small layer 184 -> 95, its kernels' time; rope_qk 121 -> 57; add_rms_norm
-// 153 -> 55; swiglu 107 -> 71, its kernels' time; the fp32 forward of B1 H12 S256
+// 153 -> 65; swiglu 107 -> 71, its kernels' time; the fp32 forward of B1 H12 S256
 // 15 -> 8): exact torch.Tensor (or Parameter) arguments on one GPU, shapes,
 // dtypes and layouts the kernels take, no dispatch or function mode, functorch
 // transform, forward-mode tangent or tracing in effect.  For anything else they
 // return None and do nothing, and the caller takes the Python operator, which
 // handles or refuses the call as always; so every error message comes from
 // there.  The nodes keep what the Python operators keep, through SavedVariable
-// (saved-tensor hooks and in-place checks apply).
+// (saved-tensor hooks and in-place checks apply; what a hook hands back is checked
+// before a kernel indexes it).
 //
 // Host code only.  The entry points of libmi_attn.so are bound by address
 // (bind()), so that this module runs whichever copy of it Python loaded.

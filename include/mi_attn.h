@@ -290,7 +290,12 @@ mi_status mi_rmsnorm_fwd(mi_dtype x_dtype, mi_dtype w_dtype, int64_t rows, int64
                          float eps, const void* x, int64_t x_row_stride, const void* weight,
                          void* y, int64_t y_row_stride, float* rstd, void* stream);
 
-/* fp32 elements of workspace mi_rmsnorm_bwd needs for this shape (0 if invalid). */
+/*
+ * fp32 elements of workspace that mi_rmsnorm_bwd runs best with for this shape
+ * (0 if invalid): one partial row of dweight per workgroup.  The least that it
+ * accepts is one per 16 rows, at most 256 (ceil(rows / 16) * hidden elements);
+ * they differ for 2048 < hidden <= 8192 only.
+ */
 int64_t mi_rmsnorm_bwd_workspace(int64_t rows, int64_t hidden);
 
 /*
@@ -300,7 +305,8 @@ int64_t mi_rmsnorm_bwd_workspace(int64_t rows, int64_t hidden);
  *   dn = dy * weight;  dx = r dn - x r^3 mean(dn * x);
  *   dweight = sum over rows of dy * round_x(x r).
  * dweight is reduced through `workspace` in a fixed order (deterministic, and
- * the same on every device).  dx may alias dy when both have the same dtype
+ * the same on every device) that depends on rows, hidden and, below the size
+ * mi_rmsnorm_bwd_workspace gives, on workspace_elems.  dx may alias dy when both have the same dtype
  * and row stride.
  */
 mi_status mi_rmsnorm_bwd(mi_dtype x_dtype, mi_dtype w_dtype, int64_t rows, int64_t hidden,
@@ -316,8 +322,8 @@ mi_status mi_rmsnorm_bwd(mi_dtype x_dtype, mi_dtype w_dtype, int64_t rows, int64
  * final norm), core/normalization.py:13-25.  Writes
  *   sum = round_x(x + res)          (x's dtype: torch's add of two such tensors)
  * and y, rstd of mi_rmsnorm_fwd over sum.  x (the residual stream), res (the
- * branch output) and sum have x's dtype; sum may alias x or res (each row is
- * read whole before any of it is written).
+ * branch output) and sum have x's dtype; sum may alias x or res (each element
+ * is read before it is written).
  */
 mi_status mi_rmsnorm_add_fwd(mi_dtype x_dtype, mi_dtype w_dtype, int64_t rows, int64_t hidden,
                              float eps, const void* x, int64_t x_row_stride, const void* res,
