@@ -58,7 +58,7 @@ def _check_every_head(q, k, v, do, causal, ref, got, what):
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("D", [16, 32, 64, 128])
 @pytest.mark.parametrize("S", [1, 31, 33, 64, 97, 128])
-def test_every_head_on_every_grid(gpu, S, D, causal):
+def test_same_heads_on_every_grid(gpu, S, D, causal):
     """Every head of a grid, whatever its size, within the rounding of the oracle
     (each head has inputs of its own); grids on one side of all lines give a head
     the same bits."""
